@@ -331,6 +331,10 @@ bool uwc_plain_fits(int cfg, int m, int n, int k, int ldc, const void* out, int 
 int uwc_gemm_plain(int cfg, const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
                    const float* b_scale, void* out, int out_mode, int ldc, hipStream_t stream);
 
+bool uwc_plain_any_fits(int n, int k, int ldc, const void* out, int out_mode, const float* b_scale, const float* res);
+int uwc_gemm_plain_any(const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
+                       const float* b_scale, const float* res, void* out, int out_mode, int ldc, hipStream_t stream);
+
 template <bool H, bool D>
 static void launch_out(int out_mode, dim3 grid, hipStream_t s, const GemmParams& p) {
   switch (out_mode) {
@@ -396,8 +400,6 @@ extern "C" int uwc_noisy_gemm(const int8_t* A, const int8_t* B, int m, int n, in
   if (flags & FLAG_PLAIN)  // checked: a plain GEMM the forced configuration takes
     return uwc_gemm_plain((flags & FLAG_PLAIN_MASK) >> FLAG_PLAIN_SHIFT, A, B, m, n, k, a_scale, b_scale, out,
                           out_mode, n, stream);
-  if (plain && m <= 64 && out_mode != OUT_NONE && !(flags & FLAG_TILE128))
-    return uwc_skinny_gemm(A, B, m, n, k, a_scale, b_scale, out, out_mode, stream);
   // 256 x 256 tiles when hashing (one tiling per nonce shape), or for a plain GEMM when they keep
   // the CUs busy: at least one tile per CU and the last round of tiles at least 90% full (2048 x
   // 12288 gives 384 tiles on 256 CUs, a half-empty second round, and runs faster on the plain
@@ -423,20 +425,24 @@ extern "C" int uwc_noisy_gemm(const int8_t* A, const int8_t* B, int m, int n, in
                                      a_scale, b_scale, out, out_mode, 0, nullptr, n, stream);
     if (st || out_mode == OUT_NONE) return st;
     const size_t es = out_mode == OUT_BF16 ? 2 : 4;
+    const float* sw_tail = b_scale ? b_scale + n256 : nullptr;
+    void* out_tail = static_cast<char*>(out) + n256 * es;
+    if (uwc_plain_any_fits(n - n256, k, n, out_tail, out_mode, sw_tail, nullptr))
+      return uwc_gemm_plain_any(A, B + (long)n256 * k, m, n - n256, k, a_scale, sw_tail, nullptr, out_tail, out_mode, n,
+                                stream);
     GemmParams q{A, B + (long)n256 * k, m, n - n256, k, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, 0,
                  a_scale, b_scale ? b_scale + n256 : nullptr, static_cast<char*>(out) + n256 * es, nullptr, n};
     const dim3 g2(((m + G_BM - 1) / G_BM) * ((n - n256 + G_BN - 1) / G_BN));
     launch_out<false, false>(out_mode, g2, stream, q);
     return uwc_launch_status("noisy_gemm (column tail)");
   }
-  // Any other plain GEMM of whole 128 x 128 tiles: the DMA-pipelined plain kernel with each
-  // step's DMA spread over the next step's passes; a 4-step ring (one workgroup per CU) when there
-  // is at most one tile per CU, else a 2-step ring (two workgroups per CU). Measured at the
-  // Qwen3-1.7B layer linears (M = 2048): the first for o and down, the second for qkv and gate_up.
+  // Every other plain GEMM with k % 128 == 0 and whole 16-byte output pieces: the plain kernels, on
+  // the form their own rule picks. Without those, small m goes to the skinny kernels.
   if (plain && !(flags & FLAG_TILE128)) {
-    const int cfg = (long)(m / 128) * (n / 128) <= cus ? 4 : 6;
-    if (uwc_plain_fits(cfg, m, n, k, n, out, out_mode, b_scale))
-      return uwc_gemm_plain(cfg, A, B, m, n, k, a_scale, b_scale, out, out_mode, n, stream);
+    if (uwc_plain_any_fits(n, k, n, out, out_mode, b_scale, nullptr))
+      return uwc_gemm_plain_any(A, B, m, n, k, a_scale, b_scale, nullptr, out, out_mode, n, stream);
+    if (m <= 64 && out_mode != OUT_NONE)
+      return uwc_skinny_gemm(A, B, m, n, k, a_scale, b_scale, out, out_mode, stream);
   }
   GemmParams p{A, B, m, n, k, r, corrA, corrB, maxabs, lmax, key, target, wins, max_wins, a_scale, b_scale, out,
                hash ? tile_dump : nullptr, n};
@@ -481,6 +487,8 @@ extern "C" int uwc_igemm_dequant_residual_f32(const int8_t* A, const int8_t* B, 
   const bool k256 = k % 128 == 0 && k <= (1 << 24) && n <= (1 << 24);
   if (m % 256 == 0 && n % 256 == 0 && k256 && fills && aligned16(Y) && aligned16(x) && n % 4 == 0)
     return uwc_gemm256_residual(A, B, m, n, k, sx, sw, x, Y, stream);
+  if (uwc_plain_any_fits(n, k, n, Y, OUT_F32, sw, x))
+    return uwc_gemm_plain_any(A, B, m, n, k, sx, sw, x, Y, OUT_F32, n, stream);
   // elsewhere: the dequantized product, then Y = fadd(x, Y) in place (each element read, then written)
   if (int st = uwc_igemm_dequant_f32(A, B, m, n, k, sx, sw, Y, stream)) return st;
   return uwc_dequant_residual(Y, nullptr, nullptr, x, m, n, Y, stream);

@@ -1,21 +1,34 @@
-// gfx950 plain int8 x int8 -> int32 GEMM (no transcript, no denoise) for the detrt linears whose
-// 256 x 256 tiles would leave CUs idle: the Qwen3-1.7B prefill linears at M = 2048 give 64-192
-// such tiles for 256 CUs. Same contract and epilogues as the plain path of uwc_noisy_gemm
-// (runtime/detrt/qwen3.py:106-126: int32 out, or fp32 / bf16 of f32(acc) * sx[i] * sw[j]).
+// gfx950 plain int8 x int8 -> int32 GEMM (no transcript, no denoise): the detrt linears and every
+// other plain product that does not fill the chip with 256 x 256 tiles, from one decoded token to a
+// prefill chunk. Same contract and epilogues as the plain path of uwc_noisy_gemm
+// (runtime/detrt/qwen3.py:106-126: int32 out, or fp32 / bf16 of f32(acc) * sx[i] * sw[j], or fp32
+// with a residual added). Two kernels, any m, n % 4 == 0, k % 128 == 0:
 //
-//   * Workgroup tile BM x BN (128 x 128 or 128 x 256), k step 128, 4 wave64s in 2 x 2, each wave
-//     a (BM / 2) x (BN / 2) block of v_mfma_i32_32x32x32_i8 (64 or 128 int32 accumulators).
+// plain_gemm_kernel, for many tiles:
+//   * Workgroup tile BM x BN (64 or 128 rows, 128 or 256 columns), k step 128, 4 wave64s in 2 x 2,
+//     each a (BM / 2) x (BN / 2) block of v_mfma_i32_32x32x32_i8.
 //   * Operands go HBM -> LDS with global_load_lds_dwordx4 into a ring of S k steps; every wave
 //     issues its share of each step (1 KiB segments, the window base in SGPRs, a fixed 32-bit
 //     lane offset), S - 1 steps ahead of the one being multiplied. One barrier per k step.
-//   * LDS rows are 128 bytes; 16-byte chunk c of tile row r sits at chunk c ^ ((r ^ (r >> 3)) & 7),
-//     so the 32-row fragment reads are conflict-free; the swizzle is applied on the global side.
 //   * Two fragment sets: the reads of pass p + 1 go out before the MFMAs of pass p.
-//   * Transposed C (the B fragment is the MFMA's first operand): lane l holds row l & 31 of a
-//     32 x 32 block and 4 consecutive columns per register group; the epilogue turns pairs of
-//     blocks around through LDS so that each store instruction writes whole row segments.
+//   * The epilogue turns pairs of blocks around through LDS so that each store instruction writes
+//     whole row segments.
+// wave_gemm_kernel, for few: small tiles whose k steps the waves of a workgroup share out (below).
+//
+// Both:
+//   * LDS rows are 128 bytes; 16-byte chunk c of tile row r sits at chunk c ^ ((r ^ (r >> 3)) & 7),
+//     so the fragment reads are conflict-free; the swizzle is applied on the global side.
+//   * Rows past m or n read the last row again and are never stored.
+//   * Transposed C (the B fragment is the MFMA's first operand): a lane holds one row of a block and
+//     4 consecutive columns per register group.
 //   * int32 sums are exact, so any tiling and k order gives the same accumulators as the other
 //     GEMM kernels of this library.
+//
+// Every shape here used to run on the register-staged 128 x 128 kernel unless its tiles were whole
+// (m, n % 128 == 0), and on the kernels of uwc_skinny.hip for m <= 64. Measured (graph-replayed,
+// fp32 dequant out, us): 777 x 12288 x 2048 69.0 -> 33.6, 777 x 2048 x 6144 63.3 -> 18.2,
+// 200 x 4096 x 2048 28.3 -> 7.0, 100 x 2048 x 6144 60.9 -> 7.3, 33 x 4096 x 14336 26.5 -> 15.0,
+// 64 x 6144 x 4096 23.9 -> 7.9, 16 x 2688 x 2560 6.4 -> 4.1, 1 x 2048 x 6144 6.3 -> 4.6.
 #include <type_traits>
 
 #include "uwc_common.h"
@@ -26,6 +39,7 @@
 #define P_OUT_I32 1
 #define P_OUT_BF16 2
 #define P_OUT_F32 3
+#define P_OUT_F32R 4  // OUT_F32 with a residual: fadd(res, fmul(fmul(f32(acc), sx), sw))
 // lambdas are always inlined: an out-of-line call would take the accumulator arrays' addresses
 #define P_AI __attribute__((always_inline))
 
@@ -39,6 +53,7 @@ struct PlainParams {
   const float* b_scale;
   void* out;
   int ldc;  // output row stride in elements
+  const float* res;  // P_OUT_F32R: the residual rows, of the output's stride
 };
 
 template <int I, int N, class F>
@@ -69,6 +84,11 @@ __device__ __forceinline__ void p_dma(u32 voff, const void* sbase, u32 lds) {
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
 }
 
+// p_dma with the non-temporal hint, for bytes read once: a weight that streams past the caches.
+__device__ __forceinline__ void p_dma_nt(u32 voff, const void* sbase, u32 lds) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
+}
+
 // Wait until at most `younger` k steps of this wave's DMA (SEG instructions each) are in flight.
 template <int SEG, int MAXY>
 __device__ __forceinline__ void p_wait_vm(int younger) {
@@ -91,7 +111,7 @@ __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
   constexpr int TA = BM * P_BK, TB = BN * P_BK;  // bytes of one stage's A and B tile
   constexpr int SA = BM / 32, SB = BN / 32;  // 1 KiB DMA segments per wave per k step
   constexpr int SEG = SA + SB;
-  static_assert(MB % 2 == 0 && NB % 2 == 0, "block parity is the row bit 5 of the swizzle");
+  static_assert(NB % 2 == 0 && (MB % 2 == 0 || MB == 1), "the epilogue takes column blocks in pairs");
   static_assert(S >= 2 && S <= 4, "ring depth");
   extern __shared__ __attribute__((aligned(1024))) u8 sm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -101,9 +121,9 @@ __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
   // in groups of 4 tile rows so that one XCD's tiles share A and B panels in its L2
   int bm0, bn0;
   {
-    const int npm = p.m / BM, npn = p.n / BN, total = npm * npn;
-    int pid = blockIdx.x;
-    if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
+    const int npm = (p.m + BM - 1) / BM, npn = (p.n + BN - 1) / BN, total = npm * npn;
+    const int xcd = blockIdx.x & 7;
+    const int pid = xcd * (total >> 3) + min(xcd, total & 7) + (int)(blockIdx.x >> 3);
     constexpr int GROUP_M = 4;
     const int grp = GROUP_M * npn, gid = pid / grp, first = gid * GROUP_M;
     const int gsz = min(npm - first, GROUP_M), in = pid - gid * grp;
@@ -118,17 +138,18 @@ __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
 
   // DMA: this wave fills segments wave SA + t of A and wave SB + t of B; lane i of a segment
   // writes LDS bytes [16 i, 16 i + 16): tile row 8 s + i / 8, physical chunk i % 8, so it
-  // fetches logical chunk (i % 8) ^ swz(row)
+  // fetches logical chunk (i % 8) ^ swz(row). Rows past the operand's last one read that one again
+  // (their products are never stored)
   u32 offa[SA], offb[SB];
 #pragma unroll
   for (int t = 0; t < SA; t++) {
     const int row = 8 * (wave * SA + t) + (lane >> 3);
-    offa[t] = (u32)((long)row * k + (((lane & 7) ^ p_swz(row)) << 4));
+    offa[t] = (u32)((long)min(row, p.m - 1 - bm0) * k + (((lane & 7) ^ p_swz(row)) << 4));
   }
 #pragma unroll
   for (int t = 0; t < SB; t++) {
     const int row = 8 * (wave * SB + t) + (lane >> 3);
-    offb[t] = (u32)((long)row * k + (((lane & 7) ^ p_swz(row)) << 4));
+    offb[t] = (u32)((long)min(row, p.n - 1 - bn0) * k + (((lane & 7) ^ p_swz(row)) << 4));
   }
   const i8* a_win = p.A + (long)bm0 * k;
   const i8* b_win = p.B + (long)bn0 * k;
@@ -147,15 +168,15 @@ __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
     issue_part(std::integral_constant<int, 0>{}, std::integral_constant<int, SEG>{}, st, k0);
   };
 
-  // fragment addresses: row (lane & 31) of a 32-row block, logical chunk 2 kp + (lane >> 5);
-  // odd blocks (row bit 5 set) flip swizzle bit 2, i.e. use pass kp ^ 2's offset
+  // fragment addresses: row (lane & 31) of the wave's first 32-row block, logical chunk 2 kp +
+  // (lane >> 5); the wave's odd blocks (row bit 5 flipped) flip swizzle bit 2, i.e. use pass
+  // kp ^ 2's offset
   u32 fa[4], fb[4];
 #pragma unroll
   for (int kp = 0; kp < 4; kp++) {
-    const int r = lane & 31, c = 2 * kp + (lane >> 5);
-    const u32 o = (u32)(r * P_BK + ((c ^ p_swz(r)) << 4));
-    fa[kp] = lds_a(0) + (u32)(wm * WM * P_BK) + o;
-    fb[kp] = lds_b(0) + (u32)(wn * WN * P_BK) + o;
+    const int ra = wm * WM + (lane & 31), rb = wn * WN + (lane & 31), c = 2 * kp + (lane >> 5);
+    fa[kp] = lds_a(0) + (u32)(ra * P_BK + ((c ^ p_swz(ra)) << 4));
+    fb[kp] = lds_b(0) + (u32)(rb * P_BK + ((c ^ p_swz(rb)) << 4));
   }
   struct Frag {
     v4i a[MB], b[NB];
@@ -252,58 +273,291 @@ __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
     u8* slot = sm + wave * 8192;
     const int hh = lane >> 5, rr = lane & 31;
     const int rj = (lane & 7) >> 1, rh = lane & 1;  // the piece a row read takes
+    // A tile that reaches past the last row or column (n % 4 == 0: four columns in or out together)
+    // takes the last operands again there, without a branch, and leaves out the store; whole tiles
+    // have a copy of the code without the tests, which cost 5% at 2048 x 12288 x 2048.
+    auto emit = [&](auto edge_c) P_AI {
+      constexpr bool EDGE = decltype(edge_c)::value;
 #pragma unroll
-    for (int i = 0; i < MB; i++) {
+      for (int i = 0; i < MB; i++) {
 #pragma unroll
-      for (int j0 = 0; j0 < NB; j0 += 2) {
+        for (int j0 = 0; j0 < NB; j0 += 2) {
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+          for (int b = 0; b < 2; b++)
 #pragma unroll
-          for (int g = 0; g < 4; g++) {
-            const v16i& v = acc[i][j0 + b];
-            *reinterpret_cast<v4i*>(slot + ((4 * b + g) * 64 + hh * 32 + (rr ^ (2 * (2 * g + hh)))) * 16) =
-                v4i{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
-          }
+            for (int g = 0; g < 4; g++) {
+              const v16i& v = acc[i][j0 + b];
+              *reinterpret_cast<v4i*>(slot + ((4 * b + g) * 64 + hh * 32 + (rr ^ (2 * (2 * g + hh)))) * 16) =
+                  v4i{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+            }
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
-          const int row0 = bm0 + wm * WM + i * 32, col = bn0 + wn * WN + (j0 + b) * 32 + 4 * (lane & 7);
-          u8* base = reinterpret_cast<u8*>(p.out) + ((long)row0 * p.ldc + col) * ES;
-          float4 sw{};
-          if constexpr (OUT != P_OUT_I32) sw = *reinterpret_cast<const float4*>(p.b_scale + col);
-          // the four LDS reads (and row scales) first, then the stores: read, wait, store in turn
-          // put an LDS round trip (and a scale load) in front of every store
-          v4i xs[4];
-          float ascs[4];
+          for (int b = 0; b < 2; b++) {
+            const int row0 = bm0 + wm * WM + i * 32, col = bn0 + wn * WN + (j0 + b) * 32 + 4 * (lane & 7);
+            u8* base = reinterpret_cast<u8*>(p.out) + ((long)row0 * p.ldc + col) * ES;
+            const int colc = EDGE ? min(col, p.n - 4) : col;
+            float4 sw{};
+            if constexpr (OUT != P_OUT_I32) sw = *reinterpret_cast<const float4*>(p.b_scale + colc);
+            // the four LDS reads (and row scales) first, then the stores: read, wait, store in turn
+            // put an LDS round trip (and a scale load) in front of every store
+            v4i xs[4];
+            float ascs[4];
+            float4 rs[4];
 #pragma unroll
-          for (int jj = 0; jj < 4; jj++) {
-            const int r = 8 * jj + (lane >> 3);
-            xs[jj] = *reinterpret_cast<const v4i*>(slot + ((4 * b + rj) * 64 + rh * 32 + (r ^ (2 * (2 * rj + rh)))) * 16);
-            if constexpr (OUT != P_OUT_I32) ascs[jj] = p.a_scale[row0 + r];
-          }
+            for (int jj = 0; jj < 4; jj++) {
+              const int r = 8 * jj + (lane >> 3);
+              xs[jj] = *reinterpret_cast<const v4i*>(slot + ((4 * b + rj) * 64 + rh * 32 + (r ^ (2 * (2 * rj + rh)))) * 16);
+              const int rowc = EDGE ? min(row0 + r, p.m - 1) : row0 + r;
+              if constexpr (OUT != P_OUT_I32) ascs[jj] = p.a_scale[rowc];
+              if constexpr (OUT == P_OUT_F32R) rs[jj] = uwc_load_nt(p.res + (long)rowc * p.ldc + colc);
+            }
 #pragma unroll
-          for (int jj = 0; jj < 4; jj++) {
-            const int r = 8 * jj + (lane >> 3);
-            const v4i x = xs[jj];
-            u8* dst = base + (long)r * p.ldc * ES;
-            if constexpr (OUT == P_OUT_I32) {
-              uwc_store_nt(dst, x);
-            } else {
-              const float asc = ascs[jj];
-              const float y0 = __fmul_rn(__fmul_rn((float)x[0], asc), sw.x);
-              const float y1 = __fmul_rn(__fmul_rn((float)x[1], asc), sw.y);
-              const float y2 = __fmul_rn(__fmul_rn((float)x[2], asc), sw.z);
-              const float y3 = __fmul_rn(__fmul_rn((float)x[3], asc), sw.w);
-              if constexpr (OUT == P_OUT_F32) {
-                uwc_store_nt(dst, float4{y0, y1, y2, y3});
+            for (int jj = 0; jj < 4; jj++) {
+              const int r = 8 * jj + (lane >> 3);
+              if (EDGE && (row0 + r >= p.m || col >= p.n)) continue;
+              const v4i x = xs[jj];
+              u8* dst = base + (long)r * p.ldc * ES;
+              if constexpr (OUT == P_OUT_I32) {
+                uwc_store_nt(dst, x);
               } else {
-                uwc_store_nt(dst, uint2{p_bf16_rne(y0) | (p_bf16_rne(y1) << 16), p_bf16_rne(y2) | (p_bf16_rne(y3) << 16)});
+                const float asc = ascs[jj];
+                const float y0 = __fmul_rn(__fmul_rn((float)x[0], asc), sw.x);
+                const float y1 = __fmul_rn(__fmul_rn((float)x[1], asc), sw.y);
+                const float y2 = __fmul_rn(__fmul_rn((float)x[2], asc), sw.z);
+                const float y3 = __fmul_rn(__fmul_rn((float)x[3], asc), sw.w);
+                if constexpr (OUT == P_OUT_F32) {
+                  uwc_store_nt(dst, float4{y0, y1, y2, y3});
+                } else if constexpr (OUT == P_OUT_F32R) {
+                  const float4 x0 = rs[jj];
+                  uwc_store_nt(dst, float4{__fadd_rn(x0.x, y0), __fadd_rn(x0.y, y1), __fadd_rn(x0.z, y2), __fadd_rn(x0.w, y3)});
+                } else {
+                  uwc_store_nt(dst, uint2{p_bf16_rne(y0) | (p_bf16_rne(y1) << 16), p_bf16_rne(y2) | (p_bf16_rne(y3) << 16)});
+                }
               }
             }
           }
         }
       }
+    };
+    if (bm0 + BM <= p.m && bn0 + BN <= p.n) emit(std::false_type{});
+    else emit(std::true_type{});
+  }
+}
+
+// A TB x TB MFMA block of int8: K8 passes of a 128-byte k step, lane l holding row l % TB and 16-byte
+// chunk CPP kp + l / TB of an operand in pass kp, and, of the transposed product, row l % TB with the
+// 16-byte pieces (four columns) 2 g + l / 32 (TB = 32, g < 4) or l / 16 (TB = 16).
+template <int TB>
+struct Mfma;
+template <>
+struct Mfma<32> {
+  typedef v16i acc_t;
+  static constexpr int PASSES = 4, G = 4;
+  static __device__ __forceinline__ v16i mul(v4i b, v4i a, v16i c) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(b, a, c, 0, 0, 0); }
+};
+template <>
+struct Mfma<16> {
+  typedef v4i acc_t;
+  static constexpr int PASSES = 2, G = 1;
+  static __device__ __forceinline__ v4i mul(v4i b, v4i a, v4i c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(b, a, c, 0, 0, 0); }
+};
+
+// The form for few tiles (decode, short prompts, narrow outputs): a workgroup of W waves owns one
+// BM x BN tile, and wave w multiplies the whole tile over the k steps w, w + W, w + 2 W, ... through
+// an LDS ring of its own (S stages), so that the waves never wait for each other until their partial
+// sums meet in LDS at the end (int32 sums are exact: the split cannot change a value). A wave reads
+// all of a step's fragments into registers, refills the stage, then multiplies.
+//   * What bounds these shapes is how many bytes are in flight from the first cycle on and, per CU,
+//     the DMA instructions of its tiles (about 26 cycles each): small tiles put every CU to work
+//     (a 2048-column product has 64 tiles of 32 columns, 128 of 16), the k split lets a workgroup
+//     ask for W S steps at once, and with no barrier in the loop a late line holds up one wave.
+//     A tile whose four waves split its rows and columns instead needs every wave's operands for
+//     each step: 100 x 2048 x 6144 takes 17.4 us on 64 x 128 tiles that way, 7.3 on 32 x 32.
+//   * ONCE (one row of tiles: every byte of B is read once): B carries the non-temporal hint, so
+//     that a weight streaming from HBM does not evict A and the scales. Weights rotated over 1.3 GB:
+//     1 x 12288 x 2048 7.0 -> 6.0 us, 1 x 4096 x 14336 12.6 -> 10.7.
+template <int BM, int BN, int TB, int W, int S, bool ONCE, int OUT>
+__global__ void __launch_bounds__(W * 64) wave_gemm_kernel(PlainParams p) {
+  typedef Mfma<TB> MM;
+  constexpr int MB = BM / TB, NB = BN / TB, NT = W * 64, NP = MM::PASSES;
+  constexpr int SA = BM / 8, SB = BN / 8, SEG = SA + SB;  // 1 KiB DMA segments per k step
+  static_assert(TB == 32 || (MB == 1 && NB <= 2), "block parity decides the swizzle");
+  constexpr int STG = (BM + BN) * P_BK;                   // bytes of one stage
+  constexpr int PC = BN / 4;                              // 16-byte pieces of a row of partial sums
+  static_assert(BM * BN * 4 <= S * STG, "a wave's partial sums reuse its ring");
+  extern __shared__ __attribute__((aligned(1024))) u8 sm[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // workgroup -> tile: contiguous runs of ids per XCD, the tile rows of a column panel of B adjacent
+  int bm0, bn0;
+  {
+    const int npm = (p.m + BM - 1) / BM, npn = (p.n + BN - 1) / BN, total = npm * npn;
+    const int xcd = blockIdx.x & 7;
+    const int pid = xcd * (total >> 3) + min(xcd, total & 7) + (int)(blockIdx.x >> 3);
+    constexpr int GROUP_M = 8;
+    const int grp = GROUP_M * npn, gid = pid / grp, first = gid * GROUP_M;
+    const int gsz = min(npm - first, GROUP_M), in = pid - gid * grp;
+    bm0 = (first + in % gsz) * BM;
+    bn0 = (in / gsz) * BN;
+  }
+  const int KT = p.k / P_BK;
+  const u32 base = __builtin_amdgcn_readfirstlane(p_lds_addr(sm) + (u32)(wave * S * STG));
+  const i8* a_win = p.A + (long)bm0 * p.k;
+  const i8* b_win = p.B + (long)bn0 * p.k;
+  u32 offa[SA], offb[SB];
+#pragma unroll
+  for (int t = 0; t < SA; t++) {
+    const int row = 8 * t + (lane >> 3);
+    offa[t] = (u32)((long)min(row, p.m - 1 - bm0) * p.k + (((lane & 7) ^ p_swz(row)) << 4));
+  }
+#pragma unroll
+  for (int t = 0; t < SB; t++) {
+    const int row = 8 * t + (lane >> 3);
+    offb[t] = (u32)((long)min(row, p.n - 1 - bn0) * p.k + (((lane & 7) ^ p_swz(row)) << 4));
+  }
+  auto issue = [&](int st, long k0) P_AI {
+    p_static_for<SEG>([&](auto dc) P_AI {
+      constexpr int d = decltype(dc)::value;
+      if constexpr (d < SA) p_dma(offa[d], a_win + k0, base + (u32)(st * STG + d * 1024));
+      else if constexpr (ONCE) p_dma_nt(offb[d - SA], b_win + k0, base + (u32)(st * STG + d * 1024));
+      else p_dma(offb[d - SA], b_win + k0, base + (u32)(st * STG + d * 1024));
+    });
+  };
+  // fragment addresses of the even and the odd blocks (the swizzle differs in the block's parity)
+  // of A in pass kp; B's rows follow A's, swizzled alike
+  u32 fa[NP][2];
+#pragma unroll
+  for (int kp = 0; kp < NP; kp++)
+#pragma unroll
+    for (int o = 0; o < 2; o++) {
+      const int r = lane % TB, c = (8 / NP) * kp + lane / TB;
+      fa[kp][o] = base + (u32)(r * P_BK + ((c ^ p_swz(r + o * TB)) << 4));
+    }
+  typename MM::acc_t acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; i++)
+#pragma unroll
+    for (int j = 0; j < NB; j++) acc[i][j] = typename MM::acc_t{};
+
+  const int steps = wave < KT ? (KT - 1 - wave) / W + 1 : 0;  // this wave's k steps
+#pragma unroll
+  for (int s = 0; s < S; s++)
+    if (s < steps) issue(s, (long)(wave + s * W) * P_BK);
+  for (int j0 = 0; j0 < steps; j0 += S) {
+    p_static_for<S>([&](auto sc) P_AI {
+      constexpr int st = decltype(sc)::value;
+      const int j = j0 + st;
+      if (j >= steps) return;
+      p_wait_vm<SEG, S - 1>(min(steps - 1 - j, S - 1));
+      v4i a[NP][MB], b[NP][NB];
+#pragma unroll
+      for (int kp = 0; kp < NP; kp++) {
+#pragma unroll
+        for (int q = 0; q < NB; q++) b[kp][q] = p_lds(fa[kp][q & 1] + (u32)(st * STG + (BM + q * TB) * P_BK));
+#pragma unroll
+        for (int i = 0; i < MB; i++) a[kp][i] = p_lds(fa[kp][i & 1] + (u32)(st * STG + i * TB * P_BK));
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (j + S < steps) issue(st, (long)(wave + (j + S) * W) * P_BK);
+#pragma unroll
+      for (int kp = 0; kp < NP; kp++)
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+          for (int q = 0; q < NB; q++) acc[i][q] = MM::mul(b[kp][q], a[kp][i], acc[i][q]);
+    });
+  }
+
+  // the partial sums: piece c4 (columns 4 c4 .. + 3) of row r at slot r PC + (c4 ^ (r % PC)) of the
+  // wave's ring (its DMA has landed and been read), so that the rows of a write and the pieces of a
+  // read fall in distinct 16-byte bank groups; then every thread adds the W copies of its pieces
+  if constexpr (OUT != P_OUT_NONE) {
+    constexpr int ES = OUT == P_OUT_BF16 ? 2 : 4;
+    u8* mine = sm + wave * S * STG;
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+      for (int q = 0; q < NB; q++)
+#pragma unroll
+        for (int g = 0; g < MM::G; g++) {
+          const int r = TB * i + lane % TB, c4 = TB / 4 * q + 2 * g + lane / TB;
+          const auto& v = acc[i][q];
+          *reinterpret_cast<v4i*>(mine + (r * PC + (c4 ^ (r & (PC - 1)))) * 16) =
+              v4i{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+        }
+    __syncthreads();
+    // past the last row or column (n % 4 == 0) the scales are the last ones again, without a branch,
+    // and only the store is left out
+    constexpr int TN = (BM * PC + NT - 1) / NT;  // pieces per thread
+    v4i xs[TN];
+    float4 sws[TN], rs[TN];
+    float ascs[TN];
+#pragma unroll
+    for (int t = 0; t < TN; t++) {
+      const int e = t * NT + tid, r = e / PC, c4 = e % PC;
+      if (TN * NT > BM * PC && e >= BM * PC) break;
+      const int row = min(bm0 + r, p.m - 1), col = min(bn0 + 4 * c4, p.n - 4);
+      if constexpr (OUT != P_OUT_I32) {
+        sws[t] = *reinterpret_cast<const float4*>(p.b_scale + col);
+        ascs[t] = p.a_scale[row];
+      }
+      if constexpr (OUT == P_OUT_F32R) rs[t] = uwc_load_nt(p.res + (long)row * p.ldc + col);
+      const u8* src = sm + (r * PC + (c4 ^ (r & (PC - 1)))) * 16;
+      xs[t] = *reinterpret_cast<const v4i*>(src);
+#pragma unroll
+      for (int w = 1; w < W; w++) xs[t] += *reinterpret_cast<const v4i*>(src + w * S * STG);
+    }
+#pragma unroll
+    for (int t = 0; t < TN; t++) {
+      const int e = t * NT + tid, r = e / PC, c4 = e % PC;
+      const int row = bm0 + r, col = bn0 + 4 * c4;
+      if ((TN * NT > BM * PC && e >= BM * PC) || row >= p.m || col >= p.n) continue;
+      const v4i x = xs[t];
+      u8* dst = reinterpret_cast<u8*>(p.out) + ((long)row * p.ldc + col) * ES;
+      if constexpr (OUT == P_OUT_I32) {
+        uwc_store_nt(dst, x);
+      } else {
+        const float4 sw = sws[t];
+        const float asc = ascs[t];
+        const float y0 = __fmul_rn(__fmul_rn((float)x[0], asc), sw.x);
+        const float y1 = __fmul_rn(__fmul_rn((float)x[1], asc), sw.y);
+        const float y2 = __fmul_rn(__fmul_rn((float)x[2], asc), sw.z);
+        const float y3 = __fmul_rn(__fmul_rn((float)x[3], asc), sw.w);
+        if constexpr (OUT == P_OUT_F32) {
+          uwc_store_nt(dst, float4{y0, y1, y2, y3});
+        } else if constexpr (OUT == P_OUT_F32R) {
+          const float4 x0 = rs[t];
+          uwc_store_nt(dst, float4{__fadd_rn(x0.x, y0), __fadd_rn(x0.y, y1), __fadd_rn(x0.z, y2), __fadd_rn(x0.w, y3)});
+        } else {
+          uwc_store_nt(dst, uint2{p_bf16_rne(y0) | (p_bf16_rne(y1) << 16), p_bf16_rne(y2) | (p_bf16_rne(y3) << 16)});
+        }
+      }
     }
   }
+}
+
+template <int BM, int BN, int TB, int W, int S, bool ONCE, int OUT>
+void wave_go(hipStream_t s, const PlainParams& p) {
+  auto kern = wave_gemm_kernel<BM, BN, TB, W, S, ONCE, OUT>;
+  constexpr int lds = W * S * (BM + BN) * P_BK;
+  static_assert(lds <= 160 * 1024, "LDS exceeds 160 KiB");
+  static bool attr = false;  // one attribute call per instantiation (the library is process-wide)
+  if (!attr) {
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    attr = true;
+  }
+  hipLaunchKernelGGL(kern, dim3(((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN)), dim3(W * 64), lds, s, p);
+}
+
+template <int BM, int BN, int TB, int W, int S>
+void wave_out(int out_mode, hipStream_t s, const PlainParams& p) {
+  const bool once = p.m <= BM;
+#define WAVE_GO(OUT) once ? wave_go<BM, BN, TB, W, S, true, OUT>(s, p) : wave_go<BM, BN, TB, W, S, false, OUT>(s, p)
+  switch (out_mode) {
+    case P_OUT_I32: WAVE_GO(P_OUT_I32); break;
+    case P_OUT_BF16: WAVE_GO(P_OUT_BF16); break;
+    case P_OUT_F32R: WAVE_GO(P_OUT_F32R); break;
+    default: WAVE_GO(P_OUT_F32); break;
+  }
+#undef WAVE_GO
 }
 
 template <int BM, int BN, int S, bool SPREAD, int OUT>
@@ -316,7 +570,7 @@ void plain_go(hipStream_t s, const PlainParams& p) {
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     attr = true;
   }
-  hipLaunchKernelGGL(kern, dim3((p.m / BM) * (p.n / BN)), dim3(P_THREADS), lds, s, p);
+  hipLaunchKernelGGL(kern, dim3(((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN)), dim3(P_THREADS), lds, s, p);
 }
 
 template <int BM, int BN, int S, bool SPREAD>
@@ -325,6 +579,7 @@ void plain_out(int out_mode, hipStream_t s, const PlainParams& p) {
     case P_OUT_NONE: plain_go<BM, BN, S, SPREAD, P_OUT_NONE>(s, p); break;
     case P_OUT_I32: plain_go<BM, BN, S, SPREAD, P_OUT_I32>(s, p); break;
     case P_OUT_BF16: plain_go<BM, BN, S, SPREAD, P_OUT_BF16>(s, p); break;
+    case P_OUT_F32R: plain_go<BM, BN, S, SPREAD, P_OUT_F32R>(s, p); break;
     default: plain_go<BM, BN, S, SPREAD, P_OUT_F32>(s, p); break;
   }
 }
@@ -355,7 +610,7 @@ int uwc_gemm_plain(int cfg, const int8_t* A, const int8_t* B, int m, int n, int 
                    const float* b_scale, void* out, int out_mode, int ldc, hipStream_t stream) {
   if (!uwc_plain_fits(cfg, m, n, k, ldc, out, out_mode, b_scale))
     return uwc_fail("uwc_gemm_plain: configuration %d does not take m=%d n=%d k=%d", cfg, m, n, k);
-  const PlainParams p{A, B, m, n, k, a_scale, b_scale, out, ldc};
+  const PlainParams p{A, B, m, n, k, a_scale, b_scale, out, ldc, nullptr};
   switch (cfg) {
     case 0: plain_out<128, 128, 4, false>(out_mode, stream, p); break;
     case 1: plain_out<128, 256, 3, false>(out_mode, stream, p); break;
@@ -365,6 +620,72 @@ int uwc_gemm_plain(int cfg, const int8_t* A, const int8_t* B, int m, int n, int 
     case 5: plain_out<128, 256, 3, true>(out_mode, stream, p); break;
     case 6: plain_out<128, 128, 2, true>(out_mode, stream, p); break;
     default: plain_out<128, 256, 2, true>(out_mode, stream, p); break;
+  }
+  return uwc_launch_status("plain_gemm");
+}
+
+// The forms the automatic choice takes, with their tile, the workgroups a CU holds at once (by LDS)
+// and the constants of their time in us: start + (k / 128) max(lat rounds, load x) + per_tile (x - 1)
+// for x tiles per CU in `rounds` rounds of `occ`. lat is what a k step of one tile takes (its wave's
+// or its barrier's chain), load what it costs a CU that has other tiles to work on, per_tile a
+// tile's share of the epilogues. Fitted to 242 shapes (m 1 .. 3000, n 1152 .. 20480, k 1152 .. 14336,
+// every form timed at each): the form with the least predicted time is on average within 1% of the
+// fastest one and within 3.4% at nine shapes of ten (16% at worst); dropping any of the nine forms
+// costs up to 29% somewhere.
+struct PlainForm {
+  int bm, bn, occ;
+  float start, lat, load, per_tile;
+};
+static const PlainForm kPlainForms[] = {
+    {128, 128, 1, 4.98f, 0.4185f, 0.0f, 7.03f},      // plain, 4-step ring
+    {128, 128, 2, 2.58f, 0.7405f, 0.0f, 6.27f},      // plain, 2-step ring
+    {64, 128, 2, 3.17f, 0.3420f, 0.3168f, 1.26f},    // plain, 3-step ring
+    {64, 64, 4, 3.17f, 0.2932f, 0.1903f, 0.50f},     // 2 waves
+    {64, 64, 2, 3.43f, 0.0f, 0.1882f, 1.05f},        // 4 waves
+    {64, 32, 1, 3.25f, 0.1306f, 0.0f, 1.65f},        // 4 waves, 2 stages
+    {32, 32, 2, 2.85f, 0.0940f, 0.0842f, 0.36f},     // 4 waves, 2 stages
+    {16, 32, 3, 2.91f, 0.0750f, 0.0622f, 0.12f},     // 4 waves, 2 stages
+    {16, 16, 3, 2.84f, 0.0541f, 0.0388f, 0.20f},     // 4 waves, 3 stages
+};
+
+static float plain_form_us(const PlainForm& f, int m, int n, int k, int cus) {
+  const long tiles = (long)((m + f.bm - 1) / f.bm) * ((n + f.bn - 1) / f.bn);
+  const long x = (tiles + cus - 1) / cus, rounds = (x + f.occ - 1) / f.occ;
+  const float step = f.lat * rounds > f.load * x ? f.lat * rounds : f.load * x;
+  return f.start + (k / P_BK) * step + f.per_tile * (x - 1);
+}
+
+// Whether uwc_gemm_plain_any takes the product: whole k steps, 16-byte output rows (and residual
+// rows), four column scales per load, 32-bit operand offsets within a tile.
+bool uwc_plain_any_fits(int n, int k, int ldc, const void* out, int out_mode, const float* b_scale, const float* res) {
+  const bool vec_out = (uintptr_t)out % 16 == 0 && ldc % 4 == 0 && n % 4 == 0 && (uintptr_t)res % 16 == 0;
+  const bool vec_scale = out_mode == P_OUT_I32 || (uintptr_t)b_scale % 16 == 0;
+  return out_mode != P_OUT_NONE && vec_out && vec_scale && k % P_BK == 0 && k >= P_BK && k <= (1 << 23);
+}
+
+// A plain GEMM of any m on the form predicted fastest; res (with P_OUT_F32): the residual, of the
+// output's row stride. Called after the argument checks of uwc_noisy_gemm and uwc_plain_any_fits.
+int uwc_gemm_plain_any(const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
+                       const float* b_scale, const float* res, void* out, int out_mode, int ldc, hipStream_t stream) {
+  const PlainParams p{A, B, m, n, k, a_scale, b_scale, out, ldc, res};
+  const int cus = uwc_cu_count();
+  int best = 0;
+  float best_us = 0.0f;
+  for (int i = 0; i < (int)(sizeof(kPlainForms) / sizeof(kPlainForms[0])); i++) {
+    const float us = plain_form_us(kPlainForms[i], m, n, k, cus);
+    if (i == 0 || us < best_us) best = i, best_us = us;
+  }
+  const int mode = res ? P_OUT_F32R : out_mode;
+  switch (best) {
+    case 0: plain_out<128, 128, 4, true>(mode, stream, p); break;
+    case 1: plain_out<128, 128, 2, true>(mode, stream, p); break;
+    case 2: plain_out<64, 128, 3, true>(mode, stream, p); break;
+    case 3: wave_out<64, 64, 32, 2, 1>(mode, stream, p); break;
+    case 4: wave_out<64, 64, 32, 4, 1>(mode, stream, p); break;
+    case 5: wave_out<64, 32, 32, 4, 2>(mode, stream, p); break;
+    case 6: wave_out<32, 32, 32, 4, 2>(mode, stream, p); break;
+    case 7: wave_out<16, 32, 16, 4, 2>(mode, stream, p); break;
+    default: wave_out<16, 16, 16, 4, 3>(mode, stream, p); break;
   }
   return uwc_launch_status("plain_gemm");
 }
