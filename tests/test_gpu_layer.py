@@ -483,3 +483,35 @@ def test_sha_row_roots_and_trace_roots(dev):
         for si in (0, 1):
             rows = [_t(r.view(np.int32), dev) for r in S.fixture_rows(d, si)]
             assert detgpu.trace_root(rows) == bytes(d[f"s{si}_root"]), (name, si)
+
+
+@pytest.mark.parametrize("rows", [3, 1500])
+@pytest.mark.parametrize("k,bs", [(8, 8), (504, 8), (520, 8), (1152, 128), (2048, 512), (2688, 128), (4104, 0), (6144, 512),
+                                  (14336, 512), (16384, 512), (16392, 8)])
+def test_quantizing_row_kernels_widths(dev, rows, k, bs):
+    """quant_act, rmsnorm_quant and swiglu_quant at the edges of their register forms (rows that end
+    inside a 512-element group, a lane's 8 elements as the whole row, one and four waves per row,
+    the longest rows held in registers and the first past them), with rows of zeros and of huge
+    values, against the oracle; the first and last rows of many."""
+    from uwc_amd import detgpu
+    if rows * k > 1 << 24:
+        rows = (1 << 24) // k
+    rng = np.random.default_rng(k + rows)
+    pick = np.r_[0:min(rows, 3), max(rows - 3, 0):rows]
+    x = rng.standard_normal((rows, k)).astype(np.float32) * np.float32(3.0)
+    x[0] = 0
+    x[rows - 1, ::3] *= np.float32(1e15)
+    q, s = detgpu.quant_act(_t(x, dev), bs)
+    rq, rs = S.quant_act(x[pick], bs)
+    assert np.array_equal(q.cpu().numpy()[pick], rq) and np.array_equal(_u32(s)[pick], _u32(rs))
+    w = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    q, s = detgpu.rmsnorm_quant(_t(x, dev), _t(w, dev), 1e-6, bs)
+    rq, rs = S.quant_act(S.det_rmsnorm(x[pick], w, np.float32(1e-6)), bs)
+    assert np.array_equal(q.cpu().numpy()[pick], rq) and np.array_equal(_u32(s)[pick], _u32(rs))
+    acc = rng.integers(-3_000_000, 3_000_000, (rows, 2 * k)).astype(np.int32)
+    s3 = rng.uniform(1e-6, 1e-4, rows).astype(np.float32)
+    sw = rng.uniform(1e-4, 1e-2, 2 * k).astype(np.float32)
+    gu = S.dequant(acc[pick], s3[pick], sw)
+    rq, rs = S.quant_act(S.det_silu(gu[:, :k]) * gu[:, k:], bs)
+    q, s = detgpu.swiglu_quant(_t(acc, dev), _t(s3, dev), _t(sw, dev), bs)
+    assert np.array_equal(q.cpu().numpy()[pick], rq) and np.array_equal(_u32(s)[pick], _u32(rs))

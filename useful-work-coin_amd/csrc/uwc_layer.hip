@@ -11,9 +11,9 @@
 //   embed_rows       the embedding gather (EMBED)
 //   rmsnorm          det_rmsnorm alone (the final-norm hidden state)
 //
-// Row kernels keep one row in LDS (one workgroup of 256 threads per row). qkv_post gives each
-// head row to one wave (head_dim 32, 64 or 128; lane d holds elements d, d + 64, ...), so its
-// reductions are wave shuffles. Every fp32 step is one correctly rounded op in the reference's
+// The quantizing row kernels keep a row in the registers of one or four waves; odd widths, wide
+// Hadamard blocks and fp32 gate | up rows keep it in LDS (one workgroup of 256 threads per row).
+// qkv_post gives four heads to a wave, one per 16-lane row. Every fp32 step is one correctly rounded op in the reference's
 // order (uwc_rows.h).
 #include "uwc_rows.h"
 
@@ -40,55 +40,94 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const float* __restrict__ 
   }
 }
 
-// quant_act (qmax 64, dx_quant_lds_g's ops) of one row held by a wave in the 8-per-lane layout of
-// fwht512_rows (lane L: elements 8 L .. 8 L + 7 of each 512-element group): the transform, the
-// row's max |y| by a wave reduction, one 8-byte store per group and lane, the scale by lane 0.
-template <int G>
-__device__ __forceinline__ void wave_quant_row(float (&y)[G][8], int lane, int lbs, i8* __restrict__ qrow,
-                                               float* __restrict__ srow) {
+// A row in the registers of W waves (W = 1: a wave has its row to itself; W = 4: the workgroup's four
+// waves share one), G 512-element groups per wave: wave w of the row holds groups w, w + W, ..., lane
+// L elements 8 L .. 8 L + 7 of each (the layout of fwht512_rows). k % 8 == 0: lanes past the row's end
+// hold zeros and neither load nor store (bs divides k, so the transform keeps them zero).
+// TAIL: the row has such lanes (without them every test of the row's end is left out: 4% of a
+// 4096 x 2048 rmsnorm_quant).
+// One wave per row needs no LDS and no barrier, and the work that does not grow with the row runs
+// once; four waves per row finish it sooner and hold a quarter of the registers each. rmsnorm_quant
+// (k = 2048, us): one wave 5.0 / 5.3 / 7.6 / 9.4 / 24.0 at 200 / 600 / 1200 / 2000 / 8192 rows, four
+// 3.9 / 5.2 / 7.4 / 10.8 / 24.5, so four below four rows per CU and for rows one wave cannot hold.
+// swiglu_quant, whose work per element is several times that, is faster on four at every size (I =
+// 6144: 18.9 -> 7.2 at 200 rows, 36.9 -> 29.2 at 2000, 124 -> 107 at 8192).
+struct RowRed {
+  float f[2][4];
+  long long l[4];
+};
+
+// max / int64 sum over the row's waves (slot: a reduction of its own of the workgroup's RowRed)
+template <int W>
+__device__ __forceinline__ float row_max(float v, RowRed& red, int slot) {
+  v = wave_max(v);
+  if constexpr (W > 1) {
+    if ((threadIdx.x & 63) == 0) red.f[slot][threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = fmaxf(fmaxf(red.f[slot][0], red.f[slot][1]), fmaxf(red.f[slot][2], red.f[slot][3]));
+  }
+  return v;
+}
+template <int W>
+__device__ __forceinline__ long long row_sum64(long long v, RowRed& red) {
+  v = wave_sum64(v);
+  if constexpr (W > 1) {
+    if ((threadIdx.x & 63) == 0) red.l[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = red.l[0] + red.l[1] + red.l[2] + red.l[3];
+  }
+  return v;
+}
+
+// quant_act (qmax 64, dx_quant_lds_g's ops) of a row held as above: the transform, the row's max
+// |y|, one 8-byte store per group and lane, the scale by the row's first lane.
+template <int G, int W, bool TAIL>
+__device__ __forceinline__ void quant_row_regs(float (&y)[G][8], int lane, int w, int k, int lbs, i8* __restrict__ qrow,
+                                               float* __restrict__ srow, RowRed& red) {
   const bool neg = fwht512_rows<G>(y, G, lane, lbs);
   float m2 = 0.f;
 #pragma unroll
   for (int g = 0; g < G; g++)
 #pragma unroll
     for (int j = 0; j < 8; j++) m2 = fmaxf(m2, fabsf(y[g][j]));
-  m2 = wave_max(m2);
+  m2 = row_max<W>(m2, red, 1);
   const float fq = 64.0f;
   const float sc = __fdiv_rn(fmaxf(m2, 1e-8f), fq);
   const double rs = neg ? -1.0 / (double)sc : 1.0 / (double)sc;  // the lane holds y or -y
-  i8* qr = qrow + lane * 8;
 #pragma unroll
   for (int g = 0; g < G; g++) {
+    const int at = (g * W + w) * 512 + lane * 8;
     u64 packed = 0;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
       const float t = fminf(fmaxf(rintf(uwc_div_rd(y[g][j], rs)), -fq), fq);
       packed |= (u64)(u8)(i8)(int)t << (8 * j);
     }
-    *reinterpret_cast<u64*>(qr + g * 512) = packed;
+    if (!TAIL || at < k) *reinterpret_cast<u64*>(qrow + at) = packed;
   }
-  if (lane == 0) *srow = lbs > 0 ? __fmul_rn(sc, __fdiv_rn(1.0f, uwc_sqrt_rn((float)(1 << lbs)))) : sc;
+  if (lane == 0 && w == 0) *srow = lbs > 0 ? __fmul_rn(sc, __fdiv_rn(1.0f, uwc_sqrt_rn((float)(1 << lbs)))) : sc;
 }
 
-// rmsnorm + quant_act with one wave per row and the row in registers, for k = 512 G (G <= 8) and
-// bs = 2^lbs <= 512: lane L holds elements 8 L .. 8 L + 7 of each 512-element group (the layout of
-// fwht512_rows), the max square and the exact fixed-point sum are wave reductions (a max and an
-// int64 sum: any order gives the same value), then the same per-element ops as dx_rmsnorm_lds and
-// dx_quant_lds_g. No LDS and no barrier: the 256-thread row kernel's five workgroup reductions
-// and LDS passes made it latency-bound (54 us per 8192 x 2048 call against 15 us of traffic).
-template <int G>
-__global__ void __launch_bounds__(256) rmsnorm_quant_wave_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                                 int rows, int lbs, float inv_d, float eps,
+// rmsnorm + quant_act of rows held in registers (k <= 512 G W, bs = 2^lbs <= 512): the max square
+// and the exact fixed-point sum are reductions whose order cannot change the value, then the same
+// per-element ops as dx_rmsnorm_lds and dx_quant_lds_g. The 256-thread LDS row kernel's five
+// workgroup reductions and LDS passes made it latency-bound (54 us per 8192 x 2048 call against 15
+// us of traffic; 25 so).
+template <int G, int W, bool TAIL>
+__global__ void __launch_bounds__(256) rmsnorm_quant_regs_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                 int rows, int k, int lbs, float inv_d, float eps,
                                                                  i8* __restrict__ q, float* __restrict__ scale) {
-  constexpr int K = 512 * G;
-  const int lane = threadIdx.x & 63;
-  const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= rows) return;  // whole waves only; no barriers below
-  const float* xr = x + r * K + lane * 8;
+  __shared__ RowRed red;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wv = W > 1 ? wave : 0;
+  const long r = W > 1 ? (long)blockIdx.x : (long)blockIdx.x * 4 + wave;
+  if (r >= rows) return;  // W = 1: whole waves, and no barriers below; W = 4: never
+  const float* xr = x + r * k;
   float y[G][8];
 #pragma unroll
   for (int g = 0; g < G; g++) {
-    const float4 a = *reinterpret_cast<const float4*>(xr + g * 512), b = *reinterpret_cast<const float4*>(xr + g * 512 + 4);
+    const int at = (g * W + wv) * 512 + lane * 8;
+    float4 a{}, b{};
+    if (!TAIL || at < k) a = *reinterpret_cast<const float4*>(xr + at), b = *reinterpret_cast<const float4*>(xr + at + 4);
     y[g][0] = a.x; y[g][1] = a.y; y[g][2] = a.z; y[g][3] = a.w;
     y[g][4] = b.x; y[g][5] = b.y; y[g][6] = b.z; y[g][7] = b.w;
   }
@@ -97,58 +136,65 @@ __global__ void __launch_bounds__(256) rmsnorm_quant_wave_kernel(const float* __
   for (int g = 0; g < G; g++)
 #pragma unroll
     for (int j = 0; j < 8; j++) mx = fmaxf(mx, __fmul_rn(y[g][j], y[g][j]));
-  mx = wave_max(mx);
-  const int sh = dx_shift(mx, dx_log2ceil(K));
+  mx = row_max<W>(mx, red, 0);
+  const int sh = dx_shift(mx, dx_log2ceil(k));
   long long acc = 0;
 #pragma unroll
   for (int g = 0; g < G; g++)
 #pragma unroll
     for (int j = 0; j < 8; j++) acc += dx_fix(__fmul_rn(y[g][j], y[g][j]), sh);
-  acc = wave_sum64(acc);
+  acc = row_sum64<W>(acc, red);
   const float ss = dx_unfix(acc, sh);
   const float rr = __fdiv_rn(1.0f, uwc_sqrt_rn(__fadd_rn(__fmul_rn(ss, inv_d), eps)));
-  const float* wr = w + lane * 8;
 #pragma unroll
   for (int g = 0; g < G; g++) {
-    const float4 a = *reinterpret_cast<const float4*>(wr + g * 512), b = *reinterpret_cast<const float4*>(wr + g * 512 + 4);
-    const float wv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    const int at = (g * W + wv) * 512 + lane * 8;
+    float4 a{}, b{};
+    if (!TAIL || at < k) a = *reinterpret_cast<const float4*>(w + at), b = *reinterpret_cast<const float4*>(w + at + 4);
+    const float wvv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-    for (int j = 0; j < 8; j++) y[g][j] = __fmul_rn(__fmul_rn(y[g][j], rr), wv[j]);
+    for (int j = 0; j < 8; j++) y[g][j] = !TAIL || at < k ? __fmul_rn(__fmul_rn(y[g][j], rr), wvv[j]) : 0.0f;
   }
-  wave_quant_row<G>(y, lane, lbs, q + r * K, scale + r);
+  quant_row_regs<G, W, TAIL>(y, lane, wv, k, lbs, q + r * k, scale + r, red);
 }
 
 // ------------------------------------------------------------------ swiglu + quant_act
-// swiglu_quant from int32 gate | up rows with one wave per row and the row in registers, for
-// I = 512 G (G <= 12) and bs <= 512: element i = fmul(silu(deq(g_i)), deq(u_i)) as in the row
-// kernel below, then wave_quant_row. No LDS and no barrier.
+// swiglu_quant from int32 gate | up rows held in the registers of four waves (I <= 2048 G, bs <=
+// 512): element i = fmul(silu(deq(g_i)), deq(u_i)) as in the LDS row kernel below, then
+// quant_row_regs. VALU-bound (det_exp and the division: about 60 instructions an element) where the
+// LDS form waited on its nine passes and barriers: I = 14336 at 2000 rows 169 -> 70 us. The test of
+// the row's end stays in whole rows too: without it the compiler loads every group before the first
+// is worked on, and the registers cost more than the tests (I = 6144 at 8192 rows 107 -> 113 us).
 template <int G>
-__global__ void __launch_bounds__(256) swiglu_quant_wave_kernel(const i32* __restrict__ acc, const float* __restrict__ s3,
-                                                                const float* __restrict__ sw, int rows, int lbs,
+__global__ void __launch_bounds__(256) swiglu_quant_regs_kernel(const i32* __restrict__ acc, const float* __restrict__ s3,
+                                                                const float* __restrict__ sw, int I, int lbs,
                                                                 i8* __restrict__ q, float* __restrict__ scale) {
-  constexpr int I = 512 * G;
-  const int lane = threadIdx.x & 63;
-  const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= rows) return;  // whole waves only; no barriers below
-  const i32* ar = acc + r * 2L * I + lane * 8;
-  const float* swr = sw + lane * 8;
+  __shared__ RowRed red;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long r = blockIdx.x;
+  const i32* ar = acc + r * 2L * I;
   const float sx = s3[r];
   float y[G][8];
 #pragma unroll
   for (int g = 0; g < G; g++) {
-    const v4i g0 = *reinterpret_cast<const v4i*>(ar + g * 512), g1 = *reinterpret_cast<const v4i*>(ar + g * 512 + 4);
-    const v4i u0 = *reinterpret_cast<const v4i*>(ar + I + g * 512), u1 = *reinterpret_cast<const v4i*>(ar + I + g * 512 + 4);
-    const float4 wg0 = *reinterpret_cast<const float4*>(swr + g * 512), wg1 = *reinterpret_cast<const float4*>(swr + g * 512 + 4);
-    const float4 wu0 = *reinterpret_cast<const float4*>(swr + I + g * 512),
-                 wu1 = *reinterpret_cast<const float4*>(swr + I + g * 512 + 4);
-    const int gv[8] = {g0[0], g0[1], g0[2], g0[3], g1[0], g1[1], g1[2], g1[3]};
-    const int uv[8] = {u0[0], u0[1], u0[2], u0[3], u1[0], u1[1], u1[2], u1[3]};
-    const float wgv[8] = {wg0.x, wg0.y, wg0.z, wg0.w, wg1.x, wg1.y, wg1.z, wg1.w};
-    const float wuv[8] = {wu0.x, wu0.y, wu0.z, wu0.w, wu1.x, wu1.y, wu1.z, wu1.w};
+    const int at = (4 * g + wave) * 512 + lane * 8;
+    if (at < I) {
+      const v4i g0 = *reinterpret_cast<const v4i*>(ar + at), g1 = *reinterpret_cast<const v4i*>(ar + at + 4);
+      const v4i u0 = *reinterpret_cast<const v4i*>(ar + I + at), u1 = *reinterpret_cast<const v4i*>(ar + I + at + 4);
+      const float4 wg0 = *reinterpret_cast<const float4*>(sw + at), wg1 = *reinterpret_cast<const float4*>(sw + at + 4);
+      const float4 wu0 = *reinterpret_cast<const float4*>(sw + I + at), wu1 = *reinterpret_cast<const float4*>(sw + I + at + 4);
+      const int gv[8] = {g0[0], g0[1], g0[2], g0[3], g1[0], g1[1], g1[2], g1[3]};
+      const int uv[8] = {u0[0], u0[1], u0[2], u0[3], u1[0], u1[1], u1[2], u1[3]};
+      const float wgv[8] = {wg0.x, wg0.y, wg0.z, wg0.w, wg1.x, wg1.y, wg1.z, wg1.w};
+      const float wuv[8] = {wu0.x, wu0.y, wu0.z, wu0.w, wu1.x, wu1.y, wu1.z, wu1.w};
 #pragma unroll
-    for (int j = 0; j < 8; j++) y[g][j] = __fmul_rn(dx_silu(dx_deq(gv[j], sx, wgv[j])), dx_deq(uv[j], sx, wuv[j]));
+      for (int j = 0; j < 8; j++) y[g][j] = __fmul_rn(dx_silu(dx_deq(gv[j], sx, wgv[j])), dx_deq(uv[j], sx, wuv[j]));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; j++) y[g][j] = 0.0f;
+    }
   }
-  wave_quant_row<G>(y, lane, lbs, q + r * (long)I, scale + r);
+  quant_row_regs<G, 4, true>(y, lane, wave, I, lbs, q + r * (long)I, scale + r, red);
 }
 
 // acc: rows x 2I (gate | up), int32 accumulators dequantized with s3[row], sw[col], or with FP
@@ -462,20 +508,21 @@ extern "C" int uwc_rmsnorm_quant_f32(const float* x, const float* w, int rows, i
   if (st) return st;
   if (rows == 0) return UWC_OK;
   const int bse = bs > 1 ? bs : 1;
-  if (k % 512 == 0 && k <= 4096 && bse <= 512 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 &&
+  if (k % 8 == 0 && k <= 16384 && bse <= 512 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 &&
       ((uintptr_t)q & 7) == 0) {
     const int lbs = __builtin_ctz((unsigned)bse);
-    const dim3 grid((unsigned)((rows + 3) / 4));
-    switch (k / 512) {
-      case 1: hipLaunchKernelGGL(rmsnorm_quant_wave_kernel<1>, grid, dim3(256), 0, stream, x, w, rows, lbs, inv_d, eps, q, scale); break;
-      case 2: hipLaunchKernelGGL(rmsnorm_quant_wave_kernel<2>, grid, dim3(256), 0, stream, x, w, rows, lbs, inv_d, eps, q, scale); break;
-      case 3: hipLaunchKernelGGL(rmsnorm_quant_wave_kernel<3>, grid, dim3(256), 0, stream, x, w, rows, lbs, inv_d, eps, q, scale); break;
-      case 4: hipLaunchKernelGGL(rmsnorm_quant_wave_kernel<4>, grid, dim3(256), 0, stream, x, w, rows, lbs, inv_d, eps, q, scale); break;
-      case 5: hipLaunchKernelGGL(rmsnorm_quant_wave_kernel<5>, grid, dim3(256), 0, stream, x, w, rows, lbs, inv_d, eps, q, scale); break;
-      case 6: hipLaunchKernelGGL(rmsnorm_quant_wave_kernel<6>, grid, dim3(256), 0, stream, x, w, rows, lbs, inv_d, eps, q, scale); break;
-      case 7: hipLaunchKernelGGL(rmsnorm_quant_wave_kernel<7>, grid, dim3(256), 0, stream, x, w, rows, lbs, inv_d, eps, q, scale); break;
-      default: hipLaunchKernelGGL(rmsnorm_quant_wave_kernel<8>, grid, dim3(256), 0, stream, x, w, rows, lbs, inv_d, eps, q, scale); break;
+#define RMSQ(G, W)                                                                                                 \
+  case G:                                                                                                          \
+    hipLaunchKernelGGL((k % (512 * W) ? rmsnorm_quant_regs_kernel<G, W, true> : rmsnorm_quant_regs_kernel<G, W, false>), \
+                       dim3(W > 1 ? (unsigned)rows : (unsigned)((rows + 3) / 4)), dim3(256), 0, stream, x, w, rows, k, \
+                       lbs, inv_d, eps, q, scale);                                                                 \
+    break;
+    if (k > 4096 || (k > 512 && rows < 4 * uwc_cu_count())) {
+      switch ((k + 2047) / 2048) { RMSQ(1, 4) RMSQ(2, 4) RMSQ(3, 4) RMSQ(4, 4) RMSQ(5, 4) RMSQ(6, 4) RMSQ(7, 4) RMSQ(8, 4) }
+    } else {
+      switch ((k + 511) / 512) { RMSQ(1, 1) RMSQ(2, 1) RMSQ(3, 1) RMSQ(4, 1) RMSQ(5, 1) RMSQ(6, 1) RMSQ(7, 1) RMSQ(8, 1) }
     }
+#undef RMSQ
     return uwc_launch_status(fn);
   }
   size_t smem;
@@ -507,17 +554,16 @@ extern "C" int uwc_swiglu_quant(const void* acc, const float* s3, const float* s
   if (st) return st;
   if (rows == 0) return UWC_OK;
   const int bse = bs > 1 ? bs : 1;
-  if (s3 && I % 512 == 0 && I <= 512 * 12 && bse <= 512 && ((uintptr_t)acc & 15) == 0 && ((uintptr_t)sw & 15) == 0 &&
+  if (s3 && I % 8 == 0 && I <= 16384 && bse <= 512 && ((uintptr_t)acc & 15) == 0 && ((uintptr_t)sw & 15) == 0 &&
       ((uintptr_t)q & 7) == 0) {
     const int lbs = __builtin_ctz((unsigned)bse);
-    const dim3 grid((unsigned)((rows + 3) / 4));
     const i32* a = static_cast<const i32*>(acc);
-#define SWQ(G)                                                                                                        \
-  case G: hipLaunchKernelGGL(swiglu_quant_wave_kernel<G>, grid, dim3(256), 0, stream, a, s3, sw, rows, lbs, q, scale); break;
-    switch (I / 512) {
-      SWQ(1) SWQ(2) SWQ(3) SWQ(4) SWQ(5) SWQ(6) SWQ(7) SWQ(8) SWQ(9) SWQ(10) SWQ(11)
-      default: hipLaunchKernelGGL(swiglu_quant_wave_kernel<12>, grid, dim3(256), 0, stream, a, s3, sw, rows, lbs, q, scale); break;
-    }
+#define SWQ(G)                                                                                                \
+  case G:                                                                                                     \
+    hipLaunchKernelGGL(swiglu_quant_regs_kernel<G>, dim3((unsigned)rows), dim3(256), 0, stream, a, s3, sw, I, \
+                       lbs, q, scale);                                                                        \
+    break;
+    switch ((I + 2047) / 2048) { SWQ(1) SWQ(2) SWQ(3) SWQ(4) SWQ(5) SWQ(6) SWQ(7) SWQ(8) }
 #undef SWQ
     return uwc_launch_status(fn);
   }

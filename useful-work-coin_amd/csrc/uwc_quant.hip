@@ -60,16 +60,13 @@ __global__ void __launch_bounds__(256) quant_act_kernel(const T* __restrict__ x,
 // with lane L ^ (h / 8): the lane holding index i (bit h clear) keeps a + b, its partner
 // keeps a - b, with a = y[i] and b = y[i + h]. Each output of a stage is one rounded add or
 // subtract of the same two inputs as in the reference's stage order, so the result is
-// bit-identical to the LDS form. With STASH the row's transformed values stay in registers
-// (k <= 512 * QA_GMAX) and every load of the row is issued before the first transform, so a
-// wave has its whole row in flight at once (one row per wave leaves few waves per SIMD at
-// M = 2048: the loads, not the occupancy, must cover the memory latency); otherwise the
-// quantizing pass reloads and transforms again.
+// bit-identical to the LDS form. The quantizing pass reloads and transforms again: the form for
+// rows too long for one group or double group per wave of a workgroup.
 #define QA_GMAX 16
 
 // one group: the lane's sign is returned as by fwht512_rows
-__device__ __forceinline__ bool fwht512(float v[8], int lane, int lbs) {
-  return fwht512_rows<1>(reinterpret_cast<float(*)[8]>(v), 1, lane, lbs);
+__device__ __forceinline__ bool fwht512(float (&v)[8], int lane, int lbs) {
+  return fwht512_rows<1>(reinterpret_cast<float(*)[8]>(&v), 1, lane, lbs);
 }
 
 __device__ __forceinline__ void load8(const float* p, float v[8]) {
@@ -88,65 +85,44 @@ __device__ __forceinline__ void load8(const uint16_t* p, float v[8]) {
   }
 }
 
-template <bool STASH, typename T>
+template <typename T>
 __global__ void __launch_bounds__(256) quant_act_wave_kernel(const T* __restrict__ x, int rows, int k, int lbs,
                                                              int qmax, i8* __restrict__ q, float* __restrict__ scale) {
   const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;  // whole waves only; no barriers below
   const int G = k >> 9;
   const T* xr = x + (u64)row * k + lane * 8;
-  float y[STASH ? QA_GMAX : 1][8];
+  float y[8];
   float mx = 0.f;
   bool neg = false;  // the lane holds the negated transform (the same for every group)
-  if constexpr (STASH) {
+  for (int g = 0; g < G; g++) {
+    load8(xr + g * 512, y);
+    neg = fwht512(y, lane, lbs);
 #pragma unroll
-    for (int g = 0; g < QA_GMAX; g++)
-      if (g < G) load8(xr + g * 512, y[g]);
-    neg = fwht512_rows<QA_GMAX>(y, G, lane, lbs);
-#pragma unroll
-    for (int g = 0; g < QA_GMAX; g++)
-      if (g < G) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) mx = fmaxf(mx, fabsf(y[g][j]));
-      }
-  } else {
-    for (int g = 0; g < G; g++) {
-      load8(xr + g * 512, y[0]);
-      neg = fwht512(y[0], lane, lbs);
-#pragma unroll
-      for (int j = 0; j < 8; j++) mx = fmaxf(mx, fabsf(y[0][j]));
-    }
+    for (int j = 0; j < 8; j++) mx = fmaxf(mx, fabsf(y[j]));
   }
   mx = wave_max(mx);
   const float fq = (float)qmax;
   const float s = __fdiv_rn(fmaxf(mx, 1e-8f), fq);
   const double rs = neg ? -1.0 / (double)s : 1.0 / (double)s;  // y / s = w * (+-1 / s)
   i8* qr = q + (u64)row * k + lane * 8;
-  auto emit = [&](const float v[8], int g) {
+  for (int g = 0; g < G; g++) {
+    load8(xr + g * 512, y);
+    fwht512(y, lane, lbs);
     u64 packed = 0;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-      const float t = fminf(fmaxf(rintf(uwc_div_rd(v[j], rs)), -fq), fq);
+      const float t = fminf(fmaxf(rintf(uwc_div_rd(y[j], rs)), -fq), fq);
       packed |= (u64)(u8)(i8)(int)t << (8 * j);
     }
     *reinterpret_cast<u64*>(qr + g * 512) = packed;
-  };
-  if constexpr (STASH) {
-#pragma unroll
-    for (int g = 0; g < QA_GMAX; g++)
-      if (g < G) emit(y[g], g);
-  } else {
-    for (int g = 0; g < G; g++) {
-      load8(xr + g * 512, y[0]);
-      fwht512(y[0], lane, lbs);
-      emit(y[0], g);
-    }
   }
   if (lane == 0) scale[row] = lbs > 0 ? __fmul_rn(s, __fdiv_rn(1.0f, uwc_sqrt_rn((float)(1 << lbs)))) : s;
 }
 
-// The same quant_act with one workgroup per row and one wave per 512-element group (k % 512 == 0,
-// k / 512 <= QA_GMAX, bs <= 512): the groups transform independently (a Hadamard block never
+// The same quant_act with one workgroup per row and one wave per 512-element group (k % 8 == 0,
+// k <= 512 QA_GMAX, bs <= 512; the last group may be partial: bs divides k, so lanes past the row's
+// end hold whole blocks of zeros and store nothing): the groups transform independently (a Hadamard block never
 // spans two groups), the waves combine their max|y| through LDS, and each quantizes its own
 // group. A row of 2048 then runs on 4 waves instead of 1: at M = 2048 the one-wave form leaves
 // half the SIMDs without a wave and the rest with one, whose dependent transform and division
@@ -158,8 +134,9 @@ __global__ void __launch_bounds__(64 * QA_GMAX) quant_act_group_kernel(const T* 
   __shared__ float wmax[QA_GMAX];
   const int lane = threadIdx.x & 63, g = threadIdx.x >> 6, G = blockDim.x >> 6;
   const u64 row = blockIdx.x;
-  float y[1][8];
-  load8(x + row * k + g * 512 + lane * 8, y[0]);
+  const bool valid = g * 512 + lane * 8 < k;
+  float y[1][8] = {};
+  if (valid) load8(x + row * k + g * 512 + lane * 8, y[0]);
   const bool neg = fwht512_rows<1>(y, 1, lane, lbs);
   float mx = 0.f;
 #pragma unroll
@@ -178,7 +155,7 @@ __global__ void __launch_bounds__(64 * QA_GMAX) quant_act_group_kernel(const T* 
     const float t = fminf(fmaxf(rintf(uwc_div_rd(y[0][j], rs)), -fq), fq);
     packed |= (u64)(u8)(i8)(int)t << (8 * j);
   }
-  *reinterpret_cast<u64*>(q + row * k + g * 512 + lane * 8) = packed;
+  if (valid) *reinterpret_cast<u64*>(q + row * k + g * 512 + lane * 8) = packed;
   if (threadIdx.x == 0) scale[row] = lbs > 0 ? __fmul_rn(s, __fdiv_rn(1.0f, uwc_sqrt_rn((float)(1 << lbs)))) : s;
 }
 
@@ -204,13 +181,13 @@ __device__ __forceinline__ void load16(const uint16_t* p, float v[16]) {
 }
 
 // quant_act in the 16-per-lane layout of uwc_fwht.h with one wave per double group and one
-// workgroup per row (k % 512 == 0,
+// workgroup per row (k % 16 == 0,
 // k <= 1024 QD_MAX, bs <= 512): a double group is 1024 elements of the row, two 512-element groups
 // split on lane bit 2, 16 consecutive elements per lane (one 64-byte run: four 16-byte loads of
 // fp32, two of bf16). The transform costs two VALU operations per element per cross-lane stage
 // instead of four; the waves combine their max|y| through LDS and each quantizes its own 1024
-// elements with one 16-byte store per lane. A group past the row's end (k / 512 odd) is held as
-// zeros and never stored. Measured against the 512-group form (graph-replayed, fp32, bs 512):
+// elements with one 16-byte store per lane. Lanes past the row's end hold zeros (whole blocks: bs
+// divides k) and never store. Measured against the 512-group form (graph-replayed, fp32, bs 512):
 // 2048 x 2048 8.96 -> 8.14 us, 2048 x 6144 19.4 -> 16.9, 8192 x 4096 50.9 -> 35.7, 8192 x 14336
 // 257 -> 134; below about two waves per SIMD (64 or 100 rows) the 512-group form is faster.
 #define QD_MAX 16
@@ -220,9 +197,9 @@ __global__ void __launch_bounds__(64 * QD_MAX) quant_act_dgroup_kernel(const T* 
                                                                        float* __restrict__ scale) {
   __shared__ float wmax[QD_MAX];
   const int lane = threadIdx.x & 63, d = threadIdx.x >> 6, D = blockDim.x >> 6;
-  const int G = k >> 9, grp = (lane >> 2) & 1;
-  const bool valid = 2 * d + grp < G;
-  const u64 off = (u64)blockIdx.x * k + d * 1024 + grp * 512 + 16 * fw16_index(lane);
+  const int at = d * 1024 + ((lane >> 2) & 1) * 512 + 16 * fw16_index(lane);
+  const bool valid = at < k;
+  const u64 off = (u64)blockIdx.x * k + at;
   float y[16];
   if (valid) {
     load16(x + off, y);
@@ -296,21 +273,26 @@ static int quant_rows(const char* fn, const T* x, int rows, int k, int bs, int q
   if (qmax < 1 || qmax > 127) return uwc_fail("%s: qmax=%d outside 1..127", fn, qmax);
   if (rows == 0) return UWC_OK;
   const int bse = bs > 1 ? bs : 1;
-  if (k % 512 == 0 && k <= 1024 * QD_MAX && bse <= 512 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)q & 15) == 0 &&
-      (long)rows * ((k + 1023) / 1024) >= 2L * 4 * uwc_cu_count()) {
-    const int lbs = 31 - __builtin_clz((unsigned)bse);
+  // Register forms, any row of whole lanes. Double groups from two waves per SIMD on (above), and
+  // where single groups would need more than 16 waves: 33 rows of 14336 took 52 us at one wave per
+  // row, 5.6 so. Rows of k % 512 != 0 (k = 2688, 9 LDS passes before): 74 rows 12.4 -> 3.1 us,
+  // 2048 rows 42 -> 11.
+  const int lbs = 31 - __builtin_clz((unsigned)bse);
+  const bool ax = ((uintptr_t)x & 15) == 0;
+  if (k % 16 == 0 && k <= 1024 * QD_MAX && bse <= 512 && ax && ((uintptr_t)q & 15) == 0 &&
+      (k > 512 * QA_GMAX || (long)rows * ((k + 1023) / 1024) >= 2L * 4 * uwc_cu_count())) {
     hipLaunchKernelGGL(quant_act_dgroup_kernel<T>, dim3((unsigned)rows), dim3(64 * ((k + 1023) / 1024)), 0, stream, x, k,
                        lbs, qmax, q, scale);
     return uwc_launch_status(fn);
   }
-  if (k % 512 == 0 && bse <= 512 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)q & 7) == 0) {
-    const int lbs = 31 - __builtin_clz((unsigned)bse);
-    const dim3 grid((unsigned)((rows + 3) / 4));
-    if (k <= 512 * QA_GMAX)
-      hipLaunchKernelGGL(quant_act_group_kernel<T>, dim3((unsigned)rows), dim3(64 * (k >> 9)), 0, stream, x, k, lbs,
-                         qmax, q, scale);
-    else
-      hipLaunchKernelGGL((quant_act_wave_kernel<false, T>), grid, dim3(256), 0, stream, x, rows, k, lbs, qmax, q, scale);
+  if (k % 8 == 0 && k <= 512 * QA_GMAX && bse <= 512 && ax && ((uintptr_t)q & 7) == 0) {
+    hipLaunchKernelGGL(quant_act_group_kernel<T>, dim3((unsigned)rows), dim3(64 * ((k + 511) / 512)), 0, stream, x, k, lbs,
+                       qmax, q, scale);
+    return uwc_launch_status(fn);
+  }
+  if (k % 512 == 0 && bse <= 512 && ax && ((uintptr_t)q & 7) == 0) {
+    hipLaunchKernelGGL(quant_act_wave_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, x, rows, k, lbs,
+                       qmax, q, scale);
     return uwc_launch_status(fn);
   }
   const size_t smem = (size_t)k * 4;
