@@ -104,7 +104,7 @@ __device__ __forceinline__ u32 p_bf16_rne(float f) {
   return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
 
-template <int BM, int BN, int S, bool SPREAD, int OUT>
+template <int BM, int BN, int S, bool SPREAD, bool RAGGED, int OUT>
 __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
   constexpr int WM = BM / 2, WN = BN / 2;  // wave block
   constexpr int MB = WM / 32, NB = WN / 32;  // 32 x 32 MFMA blocks per wave
@@ -144,12 +144,12 @@ __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
 #pragma unroll
   for (int t = 0; t < SA; t++) {
     const int row = 8 * (wave * SA + t) + (lane >> 3);
-    offa[t] = (u32)((long)min(row, p.m - 1 - bm0) * k + (((lane & 7) ^ p_swz(row)) << 4));
+    offa[t] = (u32)((long)(RAGGED ? min(row, p.m - 1 - bm0) : row) * k + (((lane & 7) ^ p_swz(row)) << 4));
   }
 #pragma unroll
   for (int t = 0; t < SB; t++) {
     const int row = 8 * (wave * SB + t) + (lane >> 3);
-    offb[t] = (u32)((long)min(row, p.n - 1 - bn0) * k + (((lane & 7) ^ p_swz(row)) << 4));
+    offb[t] = (u32)((long)(RAGGED ? min(row, p.n - 1 - bn0) : row) * k + (((lane & 7) ^ p_swz(row)) << 4));
   }
   const i8* a_win = p.A + (long)bm0 * k;
   const i8* b_win = p.B + (long)bn0 * k;
@@ -275,7 +275,8 @@ __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
     const int rj = (lane & 7) >> 1, rh = lane & 1;  // the piece a row read takes
     // A tile that reaches past the last row or column (n % 4 == 0: four columns in or out together)
     // takes the last operands again there, without a branch, and leaves out the store; whole tiles
-    // have a copy of the code without the tests, which cost 5% at 2048 x 12288 x 2048.
+    // have a copy of the code without the tests, which cost 5% at 2048 x 12288 x 2048 (and products
+    // of whole tiles only a kernel without the edge copy, whose code costs 1%).
     auto emit = [&](auto edge_c) P_AI {
       constexpr bool EDGE = decltype(edge_c)::value;
 #pragma unroll
@@ -338,7 +339,7 @@ __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
         }
       }
     };
-    if (bm0 + BM <= p.m && bn0 + BN <= p.n) emit(std::false_type{});
+    if (!RAGGED || (bm0 + BM <= p.m && bn0 + BN <= p.n)) emit(std::false_type{});
     else emit(std::true_type{});
   }
 }
@@ -560,9 +561,9 @@ void wave_out(int out_mode, hipStream_t s, const PlainParams& p) {
 #undef WAVE_GO
 }
 
-template <int BM, int BN, int S, bool SPREAD, int OUT>
+template <int BM, int BN, int S, bool SPREAD, bool RAGGED, int OUT>
 void plain_go(hipStream_t s, const PlainParams& p) {
-  auto kern = plain_gemm_kernel<BM, BN, S, SPREAD, OUT>;
+  auto kern = plain_gemm_kernel<BM, BN, S, SPREAD, RAGGED, OUT>;
   constexpr int lds = S * (BM + BN) * P_BK;
   static_assert(lds <= 160 * 1024, "LDS exceeds 160 KiB");
   static bool attr = false;  // one attribute call per instantiation (the library is process-wide)
@@ -576,11 +577,23 @@ void plain_go(hipStream_t s, const PlainParams& p) {
 template <int BM, int BN, int S, bool SPREAD>
 void plain_out(int out_mode, hipStream_t s, const PlainParams& p) {
   switch (out_mode) {
-    case P_OUT_NONE: plain_go<BM, BN, S, SPREAD, P_OUT_NONE>(s, p); break;
-    case P_OUT_I32: plain_go<BM, BN, S, SPREAD, P_OUT_I32>(s, p); break;
-    case P_OUT_BF16: plain_go<BM, BN, S, SPREAD, P_OUT_BF16>(s, p); break;
-    case P_OUT_F32R: plain_go<BM, BN, S, SPREAD, P_OUT_F32R>(s, p); break;
-    default: plain_go<BM, BN, S, SPREAD, P_OUT_F32>(s, p); break;
+    case P_OUT_NONE: plain_go<BM, BN, S, SPREAD, false, P_OUT_NONE>(s, p); break;
+    case P_OUT_I32: plain_go<BM, BN, S, SPREAD, false, P_OUT_I32>(s, p); break;
+    case P_OUT_BF16: plain_go<BM, BN, S, SPREAD, false, P_OUT_BF16>(s, p); break;
+    case P_OUT_F32R: plain_go<BM, BN, S, SPREAD, false, P_OUT_F32R>(s, p); break;
+    default: plain_go<BM, BN, S, SPREAD, false, P_OUT_F32>(s, p); break;
+  }
+}
+
+// any m, n % 4 == 0 (with an output)
+template <int BM, int BN, int S>
+void plain_any(int out_mode, hipStream_t s, const PlainParams& p) {
+  if (p.m % BM == 0 && p.n % BN == 0) return plain_out<BM, BN, S, true>(out_mode, s, p);
+  switch (out_mode) {
+    case P_OUT_I32: plain_go<BM, BN, S, true, true, P_OUT_I32>(s, p); break;
+    case P_OUT_BF16: plain_go<BM, BN, S, true, true, P_OUT_BF16>(s, p); break;
+    case P_OUT_F32R: plain_go<BM, BN, S, true, true, P_OUT_F32R>(s, p); break;
+    default: plain_go<BM, BN, S, true, true, P_OUT_F32>(s, p); break;
   }
 }
 
@@ -677,9 +690,9 @@ int uwc_gemm_plain_any(const int8_t* A, const int8_t* B, int m, int n, int k, co
   }
   const int mode = res ? P_OUT_F32R : out_mode;
   switch (best) {
-    case 0: plain_out<128, 128, 4, true>(mode, stream, p); break;
-    case 1: plain_out<128, 128, 2, true>(mode, stream, p); break;
-    case 2: plain_out<64, 128, 3, true>(mode, stream, p); break;
+    case 0: plain_any<128, 128, 4>(mode, stream, p); break;
+    case 1: plain_any<128, 128, 2>(mode, stream, p); break;
+    case 2: plain_any<64, 128, 3>(mode, stream, p); break;
     case 3: wave_out<64, 64, 32, 2, 1>(mode, stream, p); break;
     case 4: wave_out<64, 64, 32, 4, 1>(mode, stream, p); break;
     case 5: wave_out<64, 32, 32, 4, 2>(mode, stream, p); break;
