@@ -113,6 +113,13 @@ int uwc_igemm_dequant_f32(const int8_t* A, const int8_t* B, int m, int n, int k,
 int uwc_igemm_dequant_residual_f32(const int8_t* A, const int8_t* B, int m, int n, int k, const float* sx,
                                    const float* sw, const float* x, float* Y, hipStream_t stream);
 
+/* The whole linear in one call: q, scale = quant_act(x, bs) per row (uwc_quant_act_f32 with qmax 64),
+ * then Y = fmul(fmul(f32(q * W^T), scale[i]), sw[j]) (uwc_igemm_dequant_f32). x rows x k fp32, W n x k
+ * int8; q (rows x k, 16-byte aligned) and scale (rows) are the caller's scratch.
+ * Replaces DetLinear.__call__: runtime/detrt/qwen3.py:121-126. */
+int uwc_det_linear_f32(const float* x, int rows, int k, int bs, const int8_t* W, int n, const float* sw, int8_t* q,
+                       float* scale, float* Y, hipStream_t stream);
+
 /* Scratch words uwc_b3_root_and_seed needs for an input of nbytes (host-side, no GPU work). */
 int uwc_b3_scratch_words(uint64_t nbytes);
 
@@ -342,6 +349,23 @@ int uwc_embed_rows(const float* table, int64_t V, int D, const int64_t* ids, int
 #define UWC_OP_EXP 5
 #define UWC_OP_SILU 6
 int uwc_det_elementwise(int op, const float* x, const float* y, float* out, int64_t n, hipStream_t stream);
+
+/* One decoder layer in one call, the kernels of uwc_rmsnorm_quant_f32, uwc_igemm_i32, uwc_qkv_post,
+ * uwc_attention_ws (stored_exp != 0) or uwc_attention, uwc_quant_act_f32,
+ * uwc_igemm_dequant_residual_f32, uwc_rmsnorm_quant_f32, uwc_igemm_i32, uwc_swiglu_quant and
+ * uwc_igemm_dequant_residual_f32 in turn, their intermediates in scratch (at least
+ * uwc_decoder_layer_scratch_bytes, 256-byte aligned; nothing in it outlives the call's work on the
+ * stream). x and out N x D fp32 (N = B T; out may be x).
+ * Weights int8 with fp32 row scales: qkv (H + 2 Hkv) hd x D, o D x H hd, gu 2 I x D, down D x I; bs
+ * their Hadamard block sizes; q_norm, k_norm NULL with qknorm = 0.
+ * Replaces detgpu layer_fused: runtime/detgpu/stages.py:154-168. */
+uint64_t uwc_decoder_layer_scratch_bytes(int B, int T, int D, int H, int Hkv, int hd, int I, int stored_exp);
+int uwc_decoder_layer_f32(const float* x, int B, int T, int D, int H, int Hkv, int hd, int I, const float* in_norm,
+                          const float* post_norm, const float* q_norm, const float* k_norm, const float* cos_tab,
+                          const float* sin_tab, const int8_t* Wqkv, const float* sqkv, int bs_qkv, const int8_t* Wo,
+                          const float* so, int bs_o, const int8_t* Wgu, const float* sgu, int bs_gu, const int8_t* Wdown,
+                          const float* sdown, int bs_down, float inv_d, float eps, float inv_sqrt_hd, int qknorm,
+                          int stored_exp, void* scratch, uint64_t scratch_bytes, float* out, hipStream_t stream);
 
 /* ======================================================================== stage commitments
  * SHA-256 / RFC 6962 trees as runtime/detrt/stage.py:33-77: a row is little-endian 4-byte

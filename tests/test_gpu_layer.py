@@ -515,3 +515,39 @@ def test_quantizing_row_kernels_widths(dev, rows, k, bs):
     rq, rs = S.quant_act(S.det_silu(gu[:, :k]) * gu[:, k:], bs)
     q, s = detgpu.swiglu_quant(_t(acc, dev), _t(s3, dev), _t(sw, dev), bs)
     assert np.array_equal(q.cpu().numpy()[pick], rq) and np.array_equal(_u32(s)[pick], _u32(rs))
+
+
+@pytest.mark.parametrize("B,T,H,Hkv,hd,I,D,arch", [(1, 1, 2, 1, 32, 128, 64, 0), (2, 70, 4, 2, 64, 384, 256, 1),
+                                                    (1, 200, 4, 4, 128, 640, 512, 0), (3, 64, 2, 2, 32, 512, 128, 0)])
+def test_layer_call_equals_ops(dev, B, T, H, Hkv, hd, I, D, arch, monkeypatch):
+    """layer_fused as one library call equals the same layer op by op (itself pinned to the oracle):
+    ragged and whole 64-key tiles, batches, both architectures, exponentials stored or recomputed, a
+    given output and one that is x itself, and a scratch holding another call's bytes. A strided x, a
+    replaced int_gemm and a too large scratch keep their meaning."""
+    from uwc_amd import detgpu
+    cfg = dict(D=D, H=H, Hkv=Hkv, hd=hd, I=I, L=1, V=16, eps=1e-6, Bs=64, max_pos=T, theta=1e4, arch=arch)
+    m = detgpu.DetModel.random(cfg, seed=T, device=dev, with_lm_head=False)
+    L = m.layers[0]
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    for _ in range(2):
+        x = torch.randn((B * T, D), generator=g, device=dev) * 3
+        want = detgpu._layer_ops(m, L, x, B, T, None)
+        got = detgpu._layer_call(m, L, x, B, T, None)
+        assert got is not None and torch.equal(got.view(torch.int32), want.view(torch.int32))
+        monkeypatch.setattr(detgpu, "ATTN_SCRATCH_MAX", 0)
+        assert torch.equal(detgpu._layer_call(m, L, x, B, T, None), want)
+        monkeypatch.undo()
+        out = torch.empty_like(x)
+        assert detgpu.layer_fused(m, L, x, B, T, out=out) is out and torch.equal(out, want)
+    wide = torch.zeros((B * T, D + 4), device=dev)
+    wide[:, :D] = x
+    if B * T > 1:  # one row is contiguous whatever its stride
+        assert detgpu._layer_call(m, L, wide[:, :D], B, T, None) is None
+    assert torch.equal(detgpu.layer_fused(m, L, wide[:, :D], B, T), want)
+    calls = []
+    lin = L["qkv"]
+    lin.int_gemm = lambda q: (calls.append(1), type(lin).int_gemm(lin, q))[1]
+    assert torch.equal(detgpu.layer_fused(m, L, x, B, T), want) and calls == [1]
+    del lin.int_gemm
+    assert detgpu.layer_fused(m, L, x, B, T, out=x) is x and torch.equal(x, want)

@@ -648,3 +648,99 @@ extern "C" int uwc_v_transpose(const int8_t* vq, int B, int T, int Hkv, int hd, 
   hipLaunchKernelGGL(v_transpose_kernel, dim3((unsigned)N), dim3(256), 0, stream, vq, T, Hkv, hd, uwc_vt_tokens(T), vt);
   return uwc_launch_status(fn);
 }
+
+// ------------------------------------------------------------------ the whole layer
+// One host call per layer: at 200 tokens the layer's kernels take about 95 us, and queueing them one
+// Python call at a time took 125 (an allocation or two, the stream lookup and the argument
+// conversion of every op around 3 us of launch).
+namespace {
+struct LayerArena {  // byte offsets in the scratch
+  uint64_t q, s, s4, x, heads, kq, vq, qs, ks, vs, vt, oc, r1, total;
+};
+uint64_t up256(uint64_t n) { return (n + 255) & ~255ull; }
+
+LayerArena layer_arena(int B, int T, int D, int H, int Hkv, int hd, int I, int stored_exp) {
+  const uint64_t N = (uint64_t)B * T, QH = (uint64_t)H * hd, KH = (uint64_t)Hkv * hd;
+  uint64_t widest = (uint64_t)D > QH ? (uint64_t)D : QH;
+  if ((uint64_t)I > widest) widest = I;
+  // the int32 products of qkv and gate_up and the attention's exponentials follow each other: one place
+  uint64_t big = N * (QH + 2 * KH) * 4;
+  if (N * 2 * I * 4 > big) big = N * 2 * I * 4;
+  const uint64_t es = stored_exp ? uwc_attention_scratch_bytes(B, T, H) : 0;
+  if (es > big) big = es;
+  LayerArena a{};
+  uint64_t at = 0;
+  auto take = [&](uint64_t bytes) {
+    const uint64_t o = at;
+    at += up256(bytes);
+    return o;
+  };
+  a.q = take(N * widest);
+  a.s = take(N * 4);
+  a.s4 = take(N * 4);  // swiglu_quant reads gate_up's row scales and writes down's
+  a.x = take(big);
+  a.heads = take(N * QH);
+  a.kq = take(N * KH);
+  a.vq = take(N * KH);
+  a.qs = take(N * H * 4);
+  a.ks = take(N * Hkv * 4);
+  a.vs = take(N * Hkv * 4);
+  a.vt = take((uint64_t)B * KH * uwc_vt_tokens(T));
+  a.oc = take(N * QH * 4);
+  a.r1 = take(N * D * 4);
+  a.total = at;
+  return a;
+}
+}  // namespace
+
+extern "C" uint64_t uwc_decoder_layer_scratch_bytes(int B, int T, int D, int H, int Hkv, int hd, int I, int stored_exp) {
+  if (B <= 0 || T <= 0 || D <= 0 || H <= 0 || Hkv <= 0 || hd <= 0 || I <= 0) return 0;
+  return layer_arena(B, T, D, H, Hkv, hd, I, stored_exp).total;
+}
+
+extern "C" int uwc_decoder_layer_f32(const float* x, int B, int T, int D, int H, int Hkv, int hd, int I,
+                                     const float* in_norm, const float* post_norm, const float* q_norm,
+                                     const float* k_norm, const float* cos_tab, const float* sin_tab, const int8_t* Wqkv,
+                                     const float* sqkv, int bs_qkv, const int8_t* Wo, const float* so, int bs_o,
+                                     const int8_t* Wgu, const float* sgu, int bs_gu, const int8_t* Wdown,
+                                     const float* sdown, int bs_down, float inv_d, float eps, float inv_sqrt_hd,
+                                     int qknorm, int stored_exp, void* scratch, uint64_t scratch_bytes, float* out,
+                                     hipStream_t stream) {
+  const char* fn = "uwc_decoder_layer_f32";
+  if (B <= 0 || T <= 0 || D <= 0 || H <= 0 || Hkv <= 0 || hd <= 0 || I <= 0 || (int64_t)B * T > 0x7fffffff)
+    return uwc_fail("%s: bad B=%d T=%d D=%d H=%d Hkv=%d hd=%d I=%d", fn, B, T, D, H, Hkv, hd, I);
+  if (!x || !out || !scratch || ((uintptr_t)scratch & 255)) return uwc_fail("%s: null x or out, or a scratch not 256-byte aligned", fn);
+  const LayerArena a = layer_arena(B, T, D, H, Hkv, hd, I, stored_exp);
+  if (scratch_bytes < a.total)
+    return uwc_fail("%s: scratch holds %llu bytes, need %llu", fn, (unsigned long long)scratch_bytes, (unsigned long long)a.total);
+  const int N = B * T, QH = H * hd, WQ = (H + 2 * Hkv) * hd;
+  char* at = static_cast<char*>(scratch);
+  int8_t* q = reinterpret_cast<int8_t*>(at + a.q);
+  float *s = reinterpret_cast<float*>(at + a.s), *s4 = reinterpret_cast<float*>(at + a.s4);
+  int32_t* acc = reinterpret_cast<int32_t*>(at + a.x);
+  float* es = reinterpret_cast<float*>(at + a.x);
+  int8_t *qq = reinterpret_cast<int8_t*>(at + a.heads), *kq = reinterpret_cast<int8_t*>(at + a.kq),
+         *vq = reinterpret_cast<int8_t*>(at + a.vq), *vt = reinterpret_cast<int8_t*>(at + a.vt);
+  float *qs = reinterpret_cast<float*>(at + a.qs), *ks = reinterpret_cast<float*>(at + a.ks),
+        *vs = reinterpret_cast<float*>(at + a.vs), *oc = reinterpret_cast<float*>(at + a.oc),
+        *r1 = reinterpret_cast<float*>(at + a.r1);
+  int st;
+  if ((st = uwc_rmsnorm_quant_f32(x, in_norm, N, D, bs_qkv, inv_d, eps, q, s, stream))) return st;
+  if ((st = uwc_igemm_i32(q, Wqkv, N, WQ, D, acc, stream))) return st;
+  // vt's keys past T (T % 64) keep whatever the scratch held: they only meet zero probabilities
+  if ((st = uwc_qkv_post(acc, s, sqkv, q_norm, k_norm, cos_tab, sin_tab, B, T, H, Hkv, hd, eps, qknorm, qq, qs, kq, ks, vq,
+                         vs, vt, stream)))
+    return st;
+  if (stored_exp)
+    st = uwc_attention_ws(qq, qs, kq, ks, vt, vs, B, T, H, Hkv, hd, inv_sqrt_hd, oc, es,
+                          uwc_attention_scratch_bytes(B, T, H), stream);
+  else
+    st = uwc_attention(qq, qs, kq, ks, vt, vs, B, T, H, Hkv, hd, inv_sqrt_hd, oc, stream);
+  if (st) return st;
+  if ((st = uwc_quant_act_f32(oc, N, QH, bs_o, 64, q, s, stream))) return st;
+  if ((st = uwc_igemm_dequant_residual_f32(q, Wo, N, D, QH, s, so, x, r1, stream))) return st;
+  if ((st = uwc_rmsnorm_quant_f32(r1, post_norm, N, D, bs_gu, inv_d, eps, q, s, stream))) return st;
+  if ((st = uwc_igemm_i32(q, Wgu, N, 2 * I, D, acc, stream))) return st;
+  if ((st = uwc_swiglu_quant(acc, s, sgu, N, I, bs_down, q, s4, stream))) return st;
+  return uwc_igemm_dequant_residual_f32(q, Wdown, N, D, I, s4, sdown, r1, out, stream);
+}

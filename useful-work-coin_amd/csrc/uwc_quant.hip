@@ -333,3 +333,9 @@ extern "C" int uwc_dequant_f32(const int32_t* acc, const float* sx, const float*
                      sw, n, total, y);
   return uwc_launch_status("dequant");
 }
+
+extern "C" int uwc_det_linear_f32(const float* x, int rows, int k, int bs, const int8_t* W, int n, const float* sw,
+                                  int8_t* q, float* scale, float* Y, hipStream_t stream) {
+  if (int st = uwc_quant_act_f32(x, rows, k, bs, 64, q, scale, stream)) return st;
+  return uwc_igemm_dequant_f32(q, W, rows, n, k, scale, sw, Y, stream);
+}

@@ -33,8 +33,7 @@ TAG_SOUT = int.from_bytes(b"sout", "big")
 BLOCK = 1024  # bytes per committed row block (runtime/detrt/stage.py:25)
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _lib.stream
 
 
 def _f32(v: float) -> float:
@@ -218,14 +217,16 @@ def swiglu_quant(acc, s3, sw, bs: int):
 
 
 def embed(table: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
-    """table[ids] for float32 table (V, D); ids outside [0, V) raise (checked on the host)."""
+    """table[ids] for float32 table (V, D); ids outside [0, V) raise (the gather itself counts them,
+    one number read back: a min and a max first cost two reductions and two round trips)."""
     ids64 = ids.reshape(-1).to(device=table.device, dtype=torch.int64).contiguous()
     V, D = table.shape
-    if ids64.numel() and (int(ids64.min()) < 0 or int(ids64.max()) >= V):
-        raise IndexError(f"embed: token id outside [0, {V})")
     out = torch.empty((ids64.numel(), D), dtype=F32, device=table.device)
+    bad = torch.zeros(1, dtype=torch.int32, device=table.device)
     _lib.call("uwc_embed_rows", table.contiguous().data_ptr(), V, D, ids64.data_ptr(), ids64.numel(), out.data_ptr(),
-              None, _stream())
+              bad.data_ptr(), _stream())
+    if int(bad):
+        raise IndexError(f"embed: token id outside [0, {V})")
     return out
 
 
@@ -431,9 +432,61 @@ class DetModel:
         return cls(cfg, embed_t, layers, cos, sin, nw(D), lm)
 
 
+_INT_GEMM = DetLinear.int_gemm  # a layer whose linears carry another one (a miner's) runs op by op
+
+
+def _layer_call(m, L, x, B, T, out):
+    """layer_fused as one library call, or None for what that call does not take: linears that mine
+    or whose int_gemm was replaced, operands that are not contiguous float32 of the model's shapes
+    on x's device."""
+    H, Hkv, dev = m.H, m.Hkv, x.device
+    qkv, o, gu, down = L["qkv"], L["o"], L["gu"], L["down"]
+    for lin in (qkv, o, gu, down):
+        if type(lin) is not DetLinear or (lin.mine and lin.mw is not None) or \
+                getattr(lin.int_gemm, "__func__", None) is not _INT_GEMM or lin.Wq.device != dev:
+            return None
+    if x.dim() != 2 or qkv.n % (H + 2 * Hkv):
+        return None
+    N, D = x.shape
+    hd, I, qknorm = qkv.n // (H + 2 * Hkv), down.k, bool(m.qk_norm)
+    if B < 1 or T < 1 or N != B * T or (qkv.k, o.n, o.k, gu.n, gu.k, down.n) != (D, D, H * hd, 2 * I, D, D):
+        return None
+    cos, sin = L["cos"], L["sin"]
+    if cos.dim() != 2 or cos.shape[0] < T or cos.shape[1] != hd or sin.shape != cos.shape:
+        return None
+    qn, kn = (L["q_norm"], L["k_norm"]) if qknorm else (None, None)
+    ins = (x, L["in_norm"], L["post_norm"], cos, sin) + ((qn, kn) if qknorm else ())
+    for t in ins:
+        if t.dtype != F32 or t.device != dev or not t.is_contiguous():
+            return None
+    if L["in_norm"].numel() != D or L["post_norm"].numel() != D or (qknorm and (qn.numel() != hd or kn.numel() != hd)):
+        return None
+    if out is None:
+        out = torch.empty((N, D), dtype=F32, device=dev)
+    elif out.shape != (N, D) or out.dtype != F32 or not out.is_contiguous() or out.device != dev:
+        return None
+    lib = _lib.lib()
+    stored = int(0 < lib.uwc_attention_scratch_bytes(B, T, H) <= ATTN_SCRATCH_MAX)
+    nbytes = lib.uwc_decoder_layer_scratch_bytes(B, T, D, H, Hkv, hd, I, stored)
+    scratch = torch.empty(nbytes, dtype=torch.int8, device=dev)
+    _lib.call("uwc_decoder_layer_f32", x.data_ptr(), B, T, D, H, Hkv, hd, I, L["in_norm"].data_ptr(),
+              L["post_norm"].data_ptr(), qn.data_ptr() if qknorm else None, kn.data_ptr() if qknorm else None,
+              cos.data_ptr(), sin.data_ptr(), qkv.Wq.data_ptr(), qkv.sw.data_ptr(), qkv.bs, o.Wq.data_ptr(),
+              o.sw.data_ptr(), o.bs, gu.Wq.data_ptr(), gu.sw.data_ptr(), gu.bs, down.Wq.data_ptr(), down.sw.data_ptr(),
+              down.bs, 1.0 / D, m.eps, m.inv_sqrt_hd, int(qknorm), stored, scratch.data_ptr(), nbytes, out.data_ptr(),
+              _stream())
+    return out
+
+
 def layer_fused(m, L, x: torch.Tensor, B: int, T: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """One decoder layer: x (N, D) float32 -> (N, D) float32, bit-identical to detrt
     (detgpu/stages.py:154-168); out: optional (N, D) float32 destination, not overlapping x."""
+    y = _layer_call(m, L, x, B, T, out)
+    return y if y is not None else _layer_ops(m, L, x, B, T, out)
+
+
+def _layer_ops(m, L, x, B, T, out):
+    """layer_fused op by op."""
     H, Hkv = m.H, m.Hkv
     q1, s1 = rmsnorm_quant(x, L["in_norm"], m.eps, L["qkv"].bs)
     qq, qs, kq, ks, vq, vs, vt = qkv_post_vt(L["qkv"].int_gemm(q1), s1, L["qkv"].sw, L["q_norm"], L["k_norm"],

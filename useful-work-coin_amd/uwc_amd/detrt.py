@@ -13,8 +13,7 @@ from . import _lib
 from . import ops
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _lib.stream
 
 
 def hadamard_bs(hadamard_block: int, k: int) -> int:
@@ -120,12 +119,21 @@ class DetLinear:
         return ops.igemm_i32(q.contiguous(), self.Wq)
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
-        shp = x.shape
-        q, sx = quant_act(x.reshape(-1, self.k), self.bs)
+        shp, k, n = x.shape, self.k, self.n
+        flat = len(shp) == 2 and shp[1] == k
+        rows = x if flat else x.reshape(-1, k)
         if self.mine and self.mw is not None:
+            q, sx = quant_act(rows, self.bs)
             y = dequant(self.int_gemm(q), sx, self.sw)
         else:
-            y = torch.empty((q.shape[0], self.n), dtype=torch.float32, device=q.device)
-            _lib.call("uwc_igemm_dequant_f32", q.data_ptr(), self.Wq.data_ptr(), q.shape[0], self.n, self.k,
-                      sx.data_ptr(), self.sw.data_ptr(), y.data_ptr(), _stream())
-        return y.reshape(*shp[:-1], self.n)
+            rows = rows.contiguous()
+            if rows.dtype != torch.float32:
+                rows = rows.to(torch.float32)
+            m, dev = rows.shape[0], rows.device
+            y = torch.empty((m, n), dtype=torch.float32, device=dev)
+            # the quantized rows, then their scales (k % 64 == 0: both aligned)
+            scratch = torch.empty(m * (k + 4), dtype=torch.int8, device=dev)
+            q = scratch.data_ptr()
+            _lib.call("uwc_det_linear_f32", rows.data_ptr(), m, k, self.bs, self.Wq.data_ptr(), n, self.sw.data_ptr(), q,
+                      q + m * k, y.data_ptr(), _stream())
+        return y if flat else y.reshape(*shp[:-1], n)

@@ -87,8 +87,7 @@ def _p(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+_stream = _lib.stream
 
 
 assert sys.byteorder == "little", "the 32-byte values are little-endian u32 words, as the host's int32"
