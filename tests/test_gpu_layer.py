@@ -551,3 +551,20 @@ def test_layer_call_equals_ops(dev, B, T, H, Hkv, hd, I, D, arch, monkeypatch):
     assert torch.equal(detgpu.layer_fused(m, L, x, B, T), want) and calls == [1]
     del lin.int_gemm
     assert detgpu.layer_fused(m, L, x, B, T, out=x) is x and torch.equal(x, want)
+
+
+@pytest.mark.parametrize("rows,words", [(1, 5), (255, 256), (257, 300), (70, 2048), (129, 2048 + 4), (9, 16640), (3, 131073),
+                                        (2, 262144), (2, 262148)])
+def test_sha_row_roots_shapes(dev, rows, words):
+    """Row roots and tagged leaves at one block per row (many rows per workgroup), odd and even block
+    counts, a partial last block, a partial last workgroup, one row per workgroup and the longest row
+    its LDS takes, against hashlib."""
+    from uwc_amd import detgpu
+    rng = np.random.default_rng(rows + words)
+    x = rng.standard_normal((rows, words)).astype(np.float32)
+    leaves, roots = detgpu._row_leaf_words(_t(x, dev), detgpu.TAG_SOUT, 5, 7, want_roots=True)
+    got_r, got_l = detgpu.digest_bytes(roots), detgpu.digest_bytes(leaves)
+    for i in sorted({0, 1 % rows, rows // 2, rows - 1}):
+        want = S.row_root(x[i])
+        assert bytes(got_r[i]) == bytes(want)
+        assert bytes(got_l[i]) == S.tagged_leaf(b"sout", (5 + i) % 7, want)

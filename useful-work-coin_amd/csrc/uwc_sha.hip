@@ -217,127 +217,68 @@ __global__ void sha_row_leaf_kernel(u32* __restrict__ leaves, long nrows, int nb
   }
 }
 
-// The same with one quad per row (16 rows per 64-thread workgroup) for rows of at most
-// SHA_QUAD_MAXBLK blocks: the row's block leaves are copied to LDS and each level of the row tree
-// is computed by the quad's lanes, node i by lane i % 4. A lane reads both children of its node
-// inside sha_node before any lane of the wave writes a parent (the lanes issue the same
-// instructions in order, and a wave's LDS operations complete in order); a level's parent i
-// overwrites child slot i, which only parents <= i / 2 of earlier iterations read. The chain per
-// row is then log2 of the block count in node pairs instead of the block count, and a wave holds
-// 16 rows instead of 64 (4x the waves for the 8192 rows of a stage output).
-#define SHA_QUAD_MAXBLK 64
-#define SHA_QUAD_ROWS 16
-__global__ void __launch_bounds__(64) sha_row_leaf_quad_kernel(const u32* __restrict__ leaves, long nrows, int nblk,
-                                                               u32 tag, u32 base, u32 mod, u32* __restrict__ roots,
-                                                               u32* __restrict__ out) {
-  __shared__ u32 lds[SHA_QUAD_ROWS * SHA_QUAD_MAXBLK * 8];
-  const int q = threadIdx.x & 3, rl = threadIdx.x >> 2;
-  const long r = (long)blockIdx.x * SHA_QUAD_ROWS + rl;
-  const bool live = r < nrows;  // no early return: the lanes of a quad stay together
-  u32* lv = lds + rl * SHA_QUAD_MAXBLK * 8;
-  if (live)
-    for (int w = q; w < nblk * 8; w += 4) lv[w] = leaves[r * nblk * 8 + w];
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's LDS writes are done
-  __builtin_amdgcn_wave_barrier();
-  int n = nblk;
-  while (n > 1) {
-    const int half = n >> 1;
-    for (int i0 = 0; i0 < half; i0 += 4) {
-      const int i = i0 + q;
-      u32 h[8];
-      if (live && i < half) {
-        sha_node(lv + 16 * i, lv + 16 * i + 8, h);
-#pragma unroll
-        for (int k = 0; k < 8; k++) lv[8 * i + k] = h[k];
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_wave_barrier();
-    }
-    if (n & 1) {  // the odd last node moves up: words q and q + 4 by lane q
-      u32 c0 = 0, c1 = 0;
-      if (live) { c0 = lv[8 * (n - 1) + q]; c1 = lv[8 * (n - 1) + 4 + q]; }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_wave_barrier();
-      if (live) { lv[8 * half + q] = c0; lv[8 * half + 4 + q] = c1; }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_wave_barrier();
-    }
-    n = half + (n & 1);
-  }
-  if (!live || q != 0) return;
-  u32 root[8];
-#pragma unroll
-  for (int k = 0; k < 8; k++) root[k] = lv[k];
-  if (roots) {
-#pragma unroll
-    for (int k = 0; k < 8; k++) roots[r * 8 + k] = root[k];
-  }
-  if (out) {
-    u32 idx = base + (u32)r;
-    if (mod) idx %= mod;
-    u32 z[10];
-    z[0] = tag;
-    z[1] = __builtin_bswap32(idx);  // u32 little-endian bytes as a big-endian word
-#pragma unroll
-    for (int k = 0; k < 8; k++) z[2 + k] = root[k];
-    u32 h[8];
-    sha_short<10>(0u, z, h);
-#pragma unroll
-    for (int k = 0; k < 8; k++) out[r * 8 + k] = h[k];
-  }
-}
-
-// One 256-thread workgroup per row for rows of SHA_QUAD_MAXBLK .. SHA_ROWTREE_MAXBLK blocks (e.g.
-// the int32 logits rows of a 151,936-entry vocabulary: 594 blocks): the row's block leaves in LDS,
-// each level's parents computed in parallel into a second LDS buffer (an odd last node moves up),
-// then the tagged leaf. A thread per row would run its 2 (nblk - 1) compressions one after another.
+// The same with a 256-thread workgroup per `per` rows of at most SHA_ROWTREE_MAXBLK blocks: the rows'
+// block leaves in LDS, each level's parents computed in parallel over all of the rows into a second
+// buffer (an odd last node moves up), then the tagged leaves, one thread per row. A thread per row
+// would run its 2 (nblk - 1) compressions one after another. per nblk is about 512 leaves, so that
+// the first level fills the workgroup. The levels' latency (two compressions each, about 3 us for a
+// wave alone on its SIMD) bounds it. 32,768 rows of 8 blocks: 73 us with a quad of lanes per row and
+// 16 rows per wave, 34 so; rows of 594 blocks, one per workgroup, 102 at 300 rows (23 compressions
+// one after another are 70).
 #define SHA_ROWTREE_MAXBLK 1024
-__global__ void __launch_bounds__(256) sha_row_tree_kernel(const u32* __restrict__ leaves, long nrows, int nblk,
+#define SHA_ROWTREE_LEAVES 512
+__global__ void __launch_bounds__(256) sha_row_tree_kernel(const u32* __restrict__ leaves, long nrows, int nblk, int per,
                                                            u32 tag, u32 base, u32 mod, u32* __restrict__ roots,
                                                            u32* __restrict__ out) {
-  extern __shared__ u32 rt_lds[];  // two buffers of nblk x 8 words
-  const long r = blockIdx.x;
+  extern __shared__ u32 rt_lds[];  // per x nblk digests, then per x ceil(nblk / 2)
+  const int tid = threadIdx.x;
+  const long r0 = (long)blockIdx.x * per;
+  const int nr = (int)min((long)per, nrows - r0);
   u32* cur = rt_lds;
-  u32* nxt = rt_lds + nblk * 8;
-  const u32* src = leaves + r * nblk * 8;
-  for (int i = threadIdx.x; i < nblk * 8; i += blockDim.x) cur[i] = src[i];
+  u32* nxt = rt_lds + per * nblk * 8;
+  const u32* src = leaves + r0 * nblk * 8;
+  for (int i = tid; i < nr * nblk * 8; i += 256) cur[i] = src[i];
   __syncthreads();
   int n = nblk;
   while (n > 1) {
-    const int half = n >> 1;
-    for (int i = threadIdx.x; i < half; i += blockDim.x) {
+    const int half = n >> 1, up = half + (n & 1);
+    for (int e = tid; e < nr * half; e += 256) {
+      const int row = e / half, i = e - row * half;
       u32 h[8];
-      sha_node(cur + 16 * i, cur + 16 * i + 8, h);
+      sha_node(cur + (row * n + 2 * i) * 8, cur + (row * n + 2 * i + 1) * 8, h);
 #pragma unroll
-      for (int k = 0; k < 8; k++) nxt[8 * i + k] = h[k];
+      for (int k = 0; k < 8; k++) nxt[(row * up + i) * 8 + k] = h[k];
     }
-    if ((n & 1) && threadIdx.x < 8) nxt[8 * half + threadIdx.x] = cur[8 * (n - 1) + threadIdx.x];
+    if (n & 1)
+      for (int w = tid; w < nr * 8; w += 256) nxt[((w >> 3) * up + half) * 8 + (w & 7)] = cur[((w >> 3) * n + n - 1) * 8 + (w & 7)];
     __syncthreads();
     u32* t = cur;
     cur = nxt;
     nxt = t;
-    n = half + (n & 1);
+    n = up;
   }
-  if (threadIdx.x != 0) return;
-  u32 root[8];
+  for (int row = tid; row < nr; row += 256) {
+    const long r = r0 + row;
+    u32 root[8];
 #pragma unroll
-  for (int k = 0; k < 8; k++) root[k] = cur[k];
-  if (roots) {
+    for (int k = 0; k < 8; k++) root[k] = cur[row * 8 + k];
+    if (roots) {
 #pragma unroll
-    for (int k = 0; k < 8; k++) roots[r * 8 + k] = root[k];
-  }
-  if (out) {
-    u32 idx = base + (u32)r;
-    if (mod) idx %= mod;
-    u32 z[10];
-    z[0] = tag;
-    z[1] = __builtin_bswap32(idx);  // u32 little-endian bytes as a big-endian word
+      for (int k = 0; k < 8; k++) roots[r * 8 + k] = root[k];
+    }
+    if (out) {
+      u32 idx = base + (u32)r;
+      if (mod) idx %= mod;
+      u32 z[10];
+      z[0] = tag;
+      z[1] = __builtin_bswap32(idx);  // u32 little-endian bytes as a big-endian word
 #pragma unroll
-    for (int k = 0; k < 8; k++) z[2 + k] = root[k];
-    u32 h[8];
-    sha_short<10>(0u, z, h);
+      for (int k = 0; k < 8; k++) z[2 + k] = root[k];
+      u32 h[8];
+      sha_short<10>(0u, z, h);
 #pragma unroll
-    for (int k = 0; k < 8; k++) out[r * 8 + k] = h[k];
+      for (int k = 0; k < 8; k++) out[r * 8 + k] = h[k];
+    }
   }
 }
 
@@ -414,19 +355,20 @@ extern "C" int uwc_sha_row_leaves(const uint32_t* rows, int64_t nrows, int row_w
   if (scratch_words < nrows * nblk * 8)
     return uwc_fail("%s: scratch has %lld words, needs %lld", fn, (long long)scratch_words, (long long)(nrows * nblk * 8));
   const long nt = nrows * nblk;
-  const dim3 grid((unsigned)((nt + 127) / 128));
+  // four waves per workgroup, one per SIMD: with two, a CU's workgroups share two of its SIMDs (8192
+  // rows of 2048 words 90 -> 56 us, 300 of 151,936 190 -> 149)
+  const dim3 grid((unsigned)((nt + 255) / 256));
   if (row_words % 4 == 0 && ((uintptr_t)rows & 15) == 0)
-    hipLaunchKernelGGL(sha_block_leaves_kernel<true>, grid, dim3(128), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
+    hipLaunchKernelGGL(sha_block_leaves_kernel<true>, grid, dim3(256), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
   else
-    hipLaunchKernelGGL(sha_block_leaves_kernel<false>, grid, dim3(128), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
+    hipLaunchKernelGGL(sha_block_leaves_kernel<false>, grid, dim3(256), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
   int st = uwc_launch_status("sha_block_leaves");
   if (st) return st;
-  if (nblk <= SHA_QUAD_MAXBLK)
-    hipLaunchKernelGGL(sha_row_leaf_quad_kernel, dim3((unsigned)((nrows + SHA_QUAD_ROWS - 1) / SHA_QUAD_ROWS)), dim3(64),
-                       0, stream, scratch, (long)nrows, nblk, tag, index_base, index_mod, row_roots, leaves_out);
-  else if (nblk <= SHA_ROWTREE_MAXBLK && nrows <= 0x7FFFFFFFL)
-    hipLaunchKernelGGL(sha_row_tree_kernel, dim3((unsigned)nrows), dim3(256), (size_t)nblk * 64, stream, scratch,
-                       (long)nrows, nblk, tag, index_base, index_mod, row_roots, leaves_out);
+  const int per = nblk >= SHA_ROWTREE_LEAVES ? 1 : SHA_ROWTREE_LEAVES / nblk < 256 ? SHA_ROWTREE_LEAVES / nblk : 256;
+  if (nblk <= SHA_ROWTREE_MAXBLK && (nrows + per - 1) / per <= 0x7FFFFFFFL)
+    hipLaunchKernelGGL(sha_row_tree_kernel, dim3((unsigned)((nrows + per - 1) / per)), dim3(256),
+                       (size_t)per * (nblk + (nblk + 1) / 2) * 32, stream, scratch, (long)nrows, nblk, per, tag,
+                       index_base, index_mod, row_roots, leaves_out);
   else
     hipLaunchKernelGGL(sha_row_leaf_kernel, dim3((unsigned)((nrows + 63) / 64)), dim3(64), 0, stream, scratch,
                        (long)nrows, nblk, tag, index_base, index_mod, row_roots, leaves_out);
