@@ -113,6 +113,13 @@ int uwc_igemm_dequant_f32(const int8_t* A, const int8_t* B, int m, int n, int k,
 int uwc_igemm_dequant_residual_f32(const int8_t* A, const int8_t* B, int m, int n, int k, const float* sx,
                                    const float* sw, const float* x, float* Y, hipStream_t stream);
 
+/* Both C = A * B^T (int32) and Y = fmul(fmul(f32(C), sx[i]), sw[j]) (fp32), m x n each: one epilogue
+ * writes both where the 256 x 256 tiles do not take the shape, else uwc_igemm_i32 and
+ * uwc_dequant_f32; the same bits either way.
+ * Replaces DetLinear.int_gemm + dequant of the lm_head: runtime/detrt/qwen3.py:106-126, 300-311. */
+int uwc_igemm_i32_dequant_f32(const int8_t* A, const int8_t* B, int m, int n, int k, const float* sx, const float* sw,
+                              int32_t* C, float* Y, hipStream_t stream);
+
 /* The whole linear in one call: q, scale = quant_act(x, bs) per row (uwc_quant_act_f32 with qmax 64),
  * then Y = fmul(fmul(f32(q * W^T), scale[i]), sw[j]) (uwc_igemm_dequant_f32). x rows x k fp32, W n x k
  * int8; q (rows x k, 16-byte aligned) and scale (rows) are the caller's scratch.

@@ -3,7 +3,7 @@ multiples of 16, 32, 64 and 128, one column piece to many column tiles, fewer k 
 workgroup has waves and more than their rings hold, and enough tiles for every form (16 x 16 tiles
 to 128 x 128 ones with one and two workgroups per CU). int32 against the register-staged 128 x 128
 kernel (UWC_FLAG_TILE128) and, where it is cheap, the CPU oracle; the dequant epilogues (fp32, bf16,
-fp32 with a residual) bit for bit with the oracle's roundings; nothing is written past the rows."""
+fp32 beside the int32 sums, fp32 with a residual) bit for bit with the oracle's roundings; nothing is written past the rows."""
 import numpy as np
 import pytest
 import torch
@@ -57,6 +57,10 @@ def test_edges(dev, m, n, k):
     assert np.array_equal(Y.cpu().numpy().view(np.uint32), want.view(np.uint32))
     Yb = _gemm(A, B, ops.OUT_BF16, torch.empty((m, n), dtype=torch.bfloat16, device=dev), sx=sxt, sw=swt)
     assert np.array_equal(Yb.cpu().view(torch.int16).numpy().view(np.uint16), O.scale_bf16(acc, sx, sw))
+    C2, Y2 = torch.empty((m, n), dtype=torch.int32, device=dev), torch.empty((m, n), device=dev)
+    _lib.call("uwc_igemm_i32_dequant_f32", A.data_ptr(), B.data_ptr(), m, n, k, sxt.data_ptr(), swt.data_ptr(),
+              C2.data_ptr(), Y2.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(C2, ref) and torch.equal(Y2.view(torch.int32), Y.view(torch.int32))
     R = torch.full((m + 40, n), 7.0, device=dev)
     _lib.call("uwc_igemm_dequant_residual_f32", A.data_ptr(), B.data_ptr(), m, n, k, sxt.data_ptr(), swt.data_ptr(),
               xt.data_ptr(), R.data_ptr(), torch.cuda.current_stream().cuda_stream)

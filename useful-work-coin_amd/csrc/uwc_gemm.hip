@@ -331,9 +331,11 @@ bool uwc_plain_fits(int cfg, int m, int n, int k, int ldc, const void* out, int 
 int uwc_gemm_plain(int cfg, const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
                    const float* b_scale, void* out, int out_mode, int ldc, hipStream_t stream);
 
-bool uwc_plain_any_fits(int n, int k, int ldc, const void* out, int out_mode, const float* b_scale, const float* res);
+bool uwc_plain_any_fits(int n, int k, int ldc, const void* out, int out_mode, const float* b_scale, const float* res,
+                        const float* out2);
 int uwc_gemm_plain_any(const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
-                       const float* b_scale, const float* res, void* out, int out_mode, int ldc, hipStream_t stream);
+                       const float* b_scale, const float* res, void* out, float* out2, int out_mode, int ldc,
+                       hipStream_t stream);
 
 template <bool H, bool D>
 static void launch_out(int out_mode, dim3 grid, hipStream_t s, const GemmParams& p) {
@@ -427,9 +429,9 @@ extern "C" int uwc_noisy_gemm(const int8_t* A, const int8_t* B, int m, int n, in
     const size_t es = out_mode == OUT_BF16 ? 2 : 4;
     const float* sw_tail = b_scale ? b_scale + n256 : nullptr;
     void* out_tail = static_cast<char*>(out) + n256 * es;
-    if (uwc_plain_any_fits(n - n256, k, n, out_tail, out_mode, sw_tail, nullptr))
-      return uwc_gemm_plain_any(A, B + (long)n256 * k, m, n - n256, k, a_scale, sw_tail, nullptr, out_tail, out_mode, n,
-                                stream);
+    if (uwc_plain_any_fits(n - n256, k, n, out_tail, out_mode, sw_tail, nullptr, nullptr))
+      return uwc_gemm_plain_any(A, B + (long)n256 * k, m, n - n256, k, a_scale, sw_tail, nullptr, out_tail, nullptr,
+                                out_mode, n, stream);
     GemmParams q{A, B + (long)n256 * k, m, n - n256, k, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, 0,
                  a_scale, b_scale ? b_scale + n256 : nullptr, static_cast<char*>(out) + n256 * es, nullptr, n};
     const dim3 g2(((m + G_BM - 1) / G_BM) * ((n - n256 + G_BN - 1) / G_BN));
@@ -439,8 +441,8 @@ extern "C" int uwc_noisy_gemm(const int8_t* A, const int8_t* B, int m, int n, in
   // Every other plain GEMM with k % 128 == 0 and whole 16-byte output pieces: the plain kernels, on
   // the form their own rule picks. Without those, small m goes to the skinny kernels.
   if (plain && !(flags & FLAG_TILE128)) {
-    if (uwc_plain_any_fits(n, k, n, out, out_mode, b_scale, nullptr))
-      return uwc_gemm_plain_any(A, B, m, n, k, a_scale, b_scale, nullptr, out, out_mode, n, stream);
+    if (uwc_plain_any_fits(n, k, n, out, out_mode, b_scale, nullptr, nullptr))
+      return uwc_gemm_plain_any(A, B, m, n, k, a_scale, b_scale, nullptr, out, nullptr, out_mode, n, stream);
     if (m <= 64 && out_mode != OUT_NONE)
       return uwc_skinny_gemm(A, B, m, n, k, a_scale, b_scale, out, out_mode, stream);
   }
@@ -487,11 +489,32 @@ extern "C" int uwc_igemm_dequant_residual_f32(const int8_t* A, const int8_t* B, 
   const bool k256 = k % 128 == 0 && k <= (1 << 24) && n <= (1 << 24);
   if (m % 256 == 0 && n % 256 == 0 && k256 && fills && aligned16(Y) && aligned16(x) && n % 4 == 0)
     return uwc_gemm256_residual(A, B, m, n, k, sx, sw, x, Y, stream);
-  if (uwc_plain_any_fits(n, k, n, Y, OUT_F32, sw, x))
-    return uwc_gemm_plain_any(A, B, m, n, k, sx, sw, x, Y, OUT_F32, n, stream);
+  if (uwc_plain_any_fits(n, k, n, Y, OUT_F32, sw, x, nullptr))
+    return uwc_gemm_plain_any(A, B, m, n, k, sx, sw, x, Y, nullptr, OUT_F32, n, stream);
   // elsewhere: the dequantized product, then Y = fadd(x, Y) in place (each element read, then written)
   if (int st = uwc_igemm_dequant_f32(A, B, m, n, k, sx, sw, Y, stream)) return st;
   return uwc_dequant_residual(Y, nullptr, nullptr, x, m, n, Y, stream);
+}
+
+// 256 x 256 tiles over the first n / 256 * 256 columns where they fill the CUs (uwc_noisy_gemm above)
+static bool takes_large_tiles(int m, int n, int k) {
+  const int cus = uwc_cu_count();
+  const long t256 = (long)(m / 256) * (n / 256), rounds256 = (t256 + cus - 1) / cus;
+  const bool fills = n % 256 ? t256 >= 256 : t256 >= cus && t256 * 10 >= rounds256 * cus * 9;
+  return m % 256 == 0 && k % 128 == 0 && k <= (1 << 24) && n <= (1 << 24) && fills;
+}
+
+extern "C" int uwc_igemm_i32_dequant_f32(const int8_t* A, const int8_t* B, int m, int n, int k, const float* sx,
+                                         const float* sw, int32_t* C, float* Y, hipStream_t stream) {
+  const char* fn = "uwc_igemm_i32_dequant_f32";
+  if (!C || !Y) return uwc_fail("%s: null C or Y", fn);
+  if (int st = gemm_check(A, B, m, n, k, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, 0, sx, sw, Y,
+                          OUT_F32, 0))
+    return st;
+  if (!takes_large_tiles(m, n, k) && uwc_plain_any_fits(n, k, n, C, OUT_I32, sw, nullptr, Y))
+    return uwc_gemm_plain_any(A, B, m, n, k, sx, sw, nullptr, C, Y, OUT_I32, n, stream);
+  if (int st = uwc_igemm_i32(A, B, m, n, k, C, stream)) return st;
+  return uwc_dequant_f32(C, sx, sw, m, n, Y, stream);
 }
 
 int uwc_noisy_gemm256_many(int count, const int8_t* const* A, const int8_t* B, int m, int n, int k, int r,

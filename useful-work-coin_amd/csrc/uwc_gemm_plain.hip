@@ -40,6 +40,7 @@
 #define P_OUT_BF16 2
 #define P_OUT_F32 3
 #define P_OUT_F32R 4  // OUT_F32 with a residual: fadd(res, fmul(fmul(f32(acc), sx), sw))
+#define P_OUT_BOTH 5  // OUT_I32 to out and OUT_F32 to out2
 // lambdas are always inlined: an out-of-line call would take the accumulator arrays' addresses
 #define P_AI __attribute__((always_inline))
 
@@ -54,6 +55,7 @@ struct PlainParams {
   void* out;
   int ldc;  // output row stride in elements
   const float* res;  // P_OUT_F32R: the residual rows, of the output's stride
+  float* out2;       // P_OUT_BOTH: the fp32 rows, of the output's stride
 };
 
 template <int I, int N, class F>
@@ -327,6 +329,9 @@ __global__ void __launch_bounds__(P_THREADS) plain_gemm_kernel(PlainParams p) {
                 const float y3 = __fmul_rn(__fmul_rn((float)x[3], asc), sw.w);
                 if constexpr (OUT == P_OUT_F32) {
                   uwc_store_nt(dst, float4{y0, y1, y2, y3});
+                } else if constexpr (OUT == P_OUT_BOTH) {
+                  uwc_store_nt(dst, x);
+                  uwc_store_nt(p.out2 + (long)(row0 + r) * p.ldc + col, float4{y0, y1, y2, y3});
                 } else if constexpr (OUT == P_OUT_F32R) {
                   const float4 x0 = rs[jj];
                   uwc_store_nt(dst, float4{__fadd_rn(x0.x, y0), __fadd_rn(x0.y, y1), __fadd_rn(x0.z, y2), __fadd_rn(x0.w, y3)});
@@ -524,6 +529,9 @@ __global__ void __launch_bounds__(W * 64) wave_gemm_kernel(PlainParams p) {
         const float y3 = __fmul_rn(__fmul_rn((float)x[3], asc), sw.w);
         if constexpr (OUT == P_OUT_F32) {
           uwc_store_nt(dst, float4{y0, y1, y2, y3});
+        } else if constexpr (OUT == P_OUT_BOTH) {
+          uwc_store_nt(dst, x);
+          uwc_store_nt(p.out2 + (long)row * p.ldc + col, float4{y0, y1, y2, y3});
         } else if constexpr (OUT == P_OUT_F32R) {
           const float4 x0 = rs[t];
           uwc_store_nt(dst, float4{__fadd_rn(x0.x, y0), __fadd_rn(x0.y, y1), __fadd_rn(x0.z, y2), __fadd_rn(x0.w, y3)});
@@ -556,6 +564,7 @@ void wave_out(int out_mode, hipStream_t s, const PlainParams& p) {
     case P_OUT_I32: WAVE_GO(P_OUT_I32); break;
     case P_OUT_BF16: WAVE_GO(P_OUT_BF16); break;
     case P_OUT_F32R: WAVE_GO(P_OUT_F32R); break;
+    case P_OUT_BOTH: WAVE_GO(P_OUT_BOTH); break;
     default: WAVE_GO(P_OUT_F32); break;
   }
 #undef WAVE_GO
@@ -581,6 +590,7 @@ void plain_out(int out_mode, hipStream_t s, const PlainParams& p) {
     case P_OUT_I32: plain_go<BM, BN, S, SPREAD, false, P_OUT_I32>(s, p); break;
     case P_OUT_BF16: plain_go<BM, BN, S, SPREAD, false, P_OUT_BF16>(s, p); break;
     case P_OUT_F32R: plain_go<BM, BN, S, SPREAD, false, P_OUT_F32R>(s, p); break;
+    case P_OUT_BOTH: plain_go<BM, BN, S, SPREAD, false, P_OUT_BOTH>(s, p); break;
     default: plain_go<BM, BN, S, SPREAD, false, P_OUT_F32>(s, p); break;
   }
 }
@@ -593,6 +603,7 @@ void plain_any(int out_mode, hipStream_t s, const PlainParams& p) {
     case P_OUT_I32: plain_go<BM, BN, S, true, true, P_OUT_I32>(s, p); break;
     case P_OUT_BF16: plain_go<BM, BN, S, true, true, P_OUT_BF16>(s, p); break;
     case P_OUT_F32R: plain_go<BM, BN, S, true, true, P_OUT_F32R>(s, p); break;
+    case P_OUT_BOTH: plain_go<BM, BN, S, true, true, P_OUT_BOTH>(s, p); break;
     default: plain_go<BM, BN, S, true, true, P_OUT_F32>(s, p); break;
   }
 }
@@ -623,7 +634,7 @@ int uwc_gemm_plain(int cfg, const int8_t* A, const int8_t* B, int m, int n, int 
                    const float* b_scale, void* out, int out_mode, int ldc, hipStream_t stream) {
   if (!uwc_plain_fits(cfg, m, n, k, ldc, out, out_mode, b_scale))
     return uwc_fail("uwc_gemm_plain: configuration %d does not take m=%d n=%d k=%d", cfg, m, n, k);
-  const PlainParams p{A, B, m, n, k, a_scale, b_scale, out, ldc, nullptr};
+  const PlainParams p{A, B, m, n, k, a_scale, b_scale, out, ldc, nullptr, nullptr};
   switch (cfg) {
     case 0: plain_out<128, 128, 4, false>(out_mode, stream, p); break;
     case 1: plain_out<128, 256, 3, false>(out_mode, stream, p); break;
@@ -670,17 +681,20 @@ static float plain_form_us(const PlainForm& f, int m, int n, int k, int cus) {
 
 // Whether uwc_gemm_plain_any takes the product: whole k steps, 16-byte output rows (and residual
 // rows), four column scales per load, 32-bit operand offsets within a tile.
-bool uwc_plain_any_fits(int n, int k, int ldc, const void* out, int out_mode, const float* b_scale, const float* res) {
-  const bool vec_out = (uintptr_t)out % 16 == 0 && ldc % 4 == 0 && n % 4 == 0 && (uintptr_t)res % 16 == 0;
-  const bool vec_scale = out_mode == P_OUT_I32 || (uintptr_t)b_scale % 16 == 0;
+bool uwc_plain_any_fits(int n, int k, int ldc, const void* out, int out_mode, const float* b_scale, const float* res,
+                        const float* out2) {
+  const bool vec_out = (uintptr_t)out % 16 == 0 && ldc % 4 == 0 && n % 4 == 0 && (uintptr_t)res % 16 == 0 &&
+                       (uintptr_t)out2 % 16 == 0;
+  const bool vec_scale = (out_mode == P_OUT_I32 && !out2) || (uintptr_t)b_scale % 16 == 0;
   return out_mode != P_OUT_NONE && vec_out && vec_scale && k % P_BK == 0 && k >= P_BK && k <= (1 << 23);
 }
 
-// A plain GEMM of any m on the form predicted fastest; res (with P_OUT_F32): the residual, of the
-// output's row stride. Called after the argument checks of uwc_noisy_gemm and uwc_plain_any_fits.
+// A plain GEMM of any m on the form predicted fastest; res (with P_OUT_F32): the residual, out2 (with
+// P_OUT_I32): the dequantized rows beside the sums, both of the output's row stride. Called after the argument checks of uwc_noisy_gemm and uwc_plain_any_fits.
 int uwc_gemm_plain_any(const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
-                       const float* b_scale, const float* res, void* out, int out_mode, int ldc, hipStream_t stream) {
-  const PlainParams p{A, B, m, n, k, a_scale, b_scale, out, ldc, res};
+                       const float* b_scale, const float* res, void* out, float* out2, int out_mode, int ldc,
+                       hipStream_t stream) {
+  const PlainParams p{A, B, m, n, k, a_scale, b_scale, out, ldc, res, out2};
   const int cus = uwc_cu_count();
   int best = 0;
   float best_us = 0.0f;
@@ -688,7 +702,7 @@ int uwc_gemm_plain_any(const int8_t* A, const int8_t* B, int m, int n, int k, co
     const float us = plain_form_us(kPlainForms[i], m, n, k, cus);
     if (i == 0 || us < best_us) best = i, best_us = us;
   }
-  const int mode = res ? P_OUT_F32R : out_mode;
+  const int mode = res ? P_OUT_F32R : out2 ? P_OUT_BOTH : out_mode;
   switch (best) {
     case 0: plain_any<128, 128, 4>(mode, stream, p); break;
     case 1: plain_any<128, 128, 2>(mode, stream, p); break;

@@ -24,7 +24,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .detrt import DetLinear, hadamard_bs
+from .detrt import DetLinear, dequant, hadamard_bs
 from .detrt import quant_act as _quant_act
 
 F32 = torch.float32
@@ -556,7 +556,14 @@ def job_outputs(m, tokens: torch.Tensor, groups: int, upto: int | None = None) -
 def final_logits(m, x: torch.Tensor):
     """lm_head(det_rmsnorm(x, norm)) for hidden rows x (N, D): (int32 logits accumulators, fp32
     logits), the rows DetQwen3.logprobs starts from (qwen3.py:300-311)."""
-    q, s = rmsnorm_quant(x.reshape(-1, m.D), m.norm, m.eps, m.lm_head.bs)
-    acc = m.lm_head.int_gemm(q)
-    from .detrt import dequant
-    return acc, dequant(acc, s, m.lm_head.sw)
+    lin = m.lm_head
+    q, s = rmsnorm_quant(x.reshape(-1, m.D), m.norm, m.eps, lin.bs)
+    if type(lin) is not DetLinear or (lin.mine and lin.mw is not None) or \
+            getattr(lin.int_gemm, "__func__", None) is not _INT_GEMM:
+        acc = lin.int_gemm(q)
+        return acc, dequant(acc, s, lin.sw)
+    acc = torch.empty((q.shape[0], lin.n), dtype=torch.int32, device=q.device)
+    logits = torch.empty((q.shape[0], lin.n), dtype=F32, device=q.device)
+    _lib.call("uwc_igemm_i32_dequant_f32", q.data_ptr(), lin.Wq.data_ptr(), q.shape[0], lin.n, lin.k, s.data_ptr(),
+              lin.sw.data_ptr(), acc.data_ptr(), logits.data_ptr(), _stream())
+    return acc, logits
