@@ -234,6 +234,14 @@ int uwc_side_project(const int8_t* A, int m, const int8_t* EA, const int8_t* SpA
                      int8_t* corrA, int corr_a_off, int ecopy_off, const int8_t* Bp, int n, const int8_t* StA,
                      int8_t* corrB, int corr_b_off, int k, int r, int32_t* maxabs, int lmax, hipStream_t stream);
 
+/* uwc_side_project from the noise pairs themselves (PA: k words, uwc_nonce_noise's P) instead of their
+ * selection matrix, for r in {32, 64, 128}, m, n % 32 == 0, k % 128 == 0; corr offsets 0 or r
+ * (ecopy_off may be -1); A, EA, PA, ApEA, StA, StB, Bp, corrA, corrB 16-byte aligned. Same results.
+ * Replaces MinedWeight._forward's noise_rows(A) + project(A) + project(BpEBt) (ops.py:331-336). */
+int uwc_side_project_pairs(const int8_t* A, int m, const int8_t* EA, const uint32_t* PA, int8_t* ApEA, const int8_t* StB,
+                           int8_t* corrA, int corr_a_off, int ecopy_off, const int8_t* Bp, int n, const int8_t* StA,
+                           int8_t* corrB, int corr_b_off, int k, int r, int32_t* maxabs, int lmax, hipStream_t stream);
+
 /* uwc_side_project for `count` (1..32) nonces sharing the block side (StB, Bp) in one launch:
  * item i as uwc_side_project(A[i], m, EA[i], SpA[i], ApEA[i], StB, corrA[i], corr_a_off, ecopy_off,
  * Bp, n, StA[i], corrB[i], corr_b_off, k, r, maxabs[i], lmax). A, EA, SpA, ApEA, corrA, StA, corrB

@@ -548,3 +548,40 @@ def test_side_project_many_matches_oracle(dev, count, m, n, k, r):
         assert np.array_equal(it["corrA"].cpu().numpy(), wantA), i
         assert np.array_equal(it["corrB"].cpu().numpy(), wantB), i
         assert it["mx"].cpu().tolist() == [int(np.abs(X).max()), max(3, int(np.abs(Y).max()))], i
+
+
+@pytest.mark.parametrize("m,n,k,r", [(128, 192, 1536, 64), (64, 32, 128, 32), (96, 160, 640, 128), (128, 4096, 2176, 128),
+                                     (4096, 12416, 512, 64), (32, 64, 6144, 128)])
+def test_side_project_pairs_matches_oracle(dev, m, n, k, r):
+    """The operand side by roles, from the noise pairs: fewer k steps than a tile has waves and more
+    than its rings hold, a last noise block of 128 columns, 32 x 32 and 64 x 64 projection tiles.
+    maxabs is an atomic max into what the buffer held; a second call
+    gives the same bytes."""
+    ops = _ops()
+    rng = np.random.default_rng(m * 7 + n + k + r)
+    A = rng.integers(-64, 65, size=(m, k), dtype=np.int8)
+    Bp = rng.integers(-64, 65, size=(n, k), dtype=np.int8)
+    E = rng.integers(-32, 32, size=(m, r), dtype=np.int8)
+    PA = O.perm_packed(O.SEED_LABEL_A, rng.bytes(32), k, r)
+    PB = O.perm_packed(O.SEED_LABEL_B, rng.bytes(32), k, r)
+    pack = lambda P: torch.from_numpy(P.view(np.int32).copy()).to(dev)
+    L = ops.limbs_for(k)
+    StA, StB = ops.proj_matrix(pack(PA), k, r), ops.proj_matrix(pack(PB), k, r)
+    X, Y = O.project(A, PB, r), O.project(Bp, PA, r)
+    wantA = np.zeros((L, m, 2 * r), np.int8)
+    O.write_limbs(X, wantA, 0)
+    wantA[:, :, r:] = E
+    wantB = np.full((L, n, 2 * r), 7, np.int8)
+    O.write_limbs(Y, wantB, r)
+    Ad, Bd = torch.from_numpy(A).to(dev), torch.from_numpy(Bp).to(dev)
+    for call in range(2):
+        ApEA = torch.empty_like(Ad)
+        corrA = torch.zeros((L, m, 2 * r), dtype=torch.int8, device=dev)
+        corrB = torch.full((L, n, 2 * r), 7, dtype=torch.int8, device=dev)
+        mx = torch.tensor([0, 3], dtype=torch.int32, device=dev)
+        ops.side_project_pairs(Ad, torch.from_numpy(E).to(dev), pack(PA), ApEA, StB, corrA, Bd, StA, corrB, maxabs=mx,
+                               corr_a_off=0, ecopy_off=r, corr_b_off=r)
+        assert np.array_equal(ApEA.cpu().numpy(), O.noise_apply(A, E, PA)), call
+        assert np.array_equal(corrA.cpu().numpy(), wantA), call
+        assert np.array_equal(corrB.cpu().numpy(), wantB), call
+        assert mx.cpu().tolist() == [int(np.abs(X).max()), max(3, int(np.abs(Y).max()))], call
