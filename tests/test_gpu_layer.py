@@ -554,11 +554,11 @@ def test_layer_call_equals_ops(dev, B, T, H, Hkv, hd, I, D, arch, monkeypatch):
 
 
 @pytest.mark.parametrize("rows,words", [(1, 5), (255, 256), (257, 300), (70, 2048), (129, 2048 + 4), (9, 16640), (3, 131073),
-                                        (2, 262144), (2, 262148)])
+                                        (2, 262144), (2, 262148), (1025, 4096), (1500, 4098), (2100, 4096)])
 def test_sha_row_roots_shapes(dev, rows, words):
     """Row roots and tagged leaves at one block per row (many rows per workgroup), odd and even block
-    counts, a partial last block, a partial last workgroup, one row per workgroup and the longest row
-    its LDS takes, against hashlib."""
+    counts, a partial last block, a partial last workgroup, one row per workgroup, the longest row its LDS
+    takes, and block leaves just past one and two waves per CU, against hashlib."""
     from uwc_amd import detgpu
     rng = np.random.default_rng(rows + words)
     x = rng.standard_normal((rows, words)).astype(np.float32)

@@ -356,12 +356,16 @@ extern "C" int uwc_sha_row_leaves(const uint32_t* rows, int64_t nrows, int row_w
     return uwc_fail("%s: scratch has %lld words, needs %lld", fn, (long long)scratch_words, (long long)(nrows * nblk * 8));
   const long nt = nrows * nblk;
   // four waves per workgroup, one per SIMD: with two, a CU's workgroups share two of its SIMDs (8192
-  // rows of 2048 words 90 -> 56 us, 300 of 151,936 190 -> 149)
-  const dim3 grid((unsigned)((nt + 255) / 256));
+  // rows of 2048 words 90 -> 56 us, 300 of 151,936 190 -> 149). While the waves are no more than one
+  // or two per CU, workgroups of one or two spread them over the CUs (186 and 372 waves, 20 and 40 rows
+  // of 151,936: 57.2 -> 55.7 us; logits of 20 rows with their roots 198 -> 196, of 6 rows 186 -> 184)
+  const long waves = (nt + 63) / 64, cus = uwc_cu_count();
+  const int threads = waves <= cus ? 64 : waves <= 2 * cus ? 128 : 256;
+  const dim3 grid((unsigned)((nt + threads - 1) / threads));
   if (row_words % 4 == 0 && ((uintptr_t)rows & 15) == 0)
-    hipLaunchKernelGGL(sha_block_leaves_kernel<true>, grid, dim3(256), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
+    hipLaunchKernelGGL(sha_block_leaves_kernel<true>, grid, dim3(threads), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
   else
-    hipLaunchKernelGGL(sha_block_leaves_kernel<false>, grid, dim3(256), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
+    hipLaunchKernelGGL(sha_block_leaves_kernel<false>, grid, dim3(threads), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
   int st = uwc_launch_status("sha_block_leaves");
   if (st) return st;
   const int per = nblk >= SHA_ROWTREE_LEAVES ? 1 : SHA_ROWTREE_LEAVES / nblk < 256 ? SHA_ROWTREE_LEAVES / nblk : 256;
