@@ -568,3 +568,19 @@ def test_sha_row_roots_shapes(dev, rows, words):
         want = S.row_root(x[i])
         assert bytes(got_r[i]) == bytes(want)
         assert bytes(got_l[i]) == S.tagged_leaf(b"sout", (5 + i) % 7, want)
+
+
+@pytest.mark.parametrize("op,rows,k", [("quant", (1 << 26) + 3, 8), ("quant", (1 << 26) + 3, 16), ("quant", (1 << 24) + 3, 9)])
+def test_row_kernels_past_one_launch(dev, op, rows, k):
+    """More rows than one launch of a workgroup per row may hold (2^32 threads): every row as in calls
+    over the halves, which fit."""
+    from uwc_amd import detgpu
+    g = torch.Generator(device=dev)
+    g.manual_seed(k)
+    x = torch.randn((rows, k), device=dev, generator=g)
+    run = lambda a, b: detgpu.quant_act(x[a:b], k & -k)
+    q, s = run(0, rows)
+    h = rows // 2
+    for a, b in ((0, h), (h, rows)):
+        qh, sh = run(a, b)
+        assert torch.equal(q[a:b], qh) and torch.equal(s[a:b].view(torch.int32), sh.view(torch.int32))

@@ -56,6 +56,18 @@ int uwc_launch_status(const char* kernel);
 // Compute units of the current device (cached per device).
 int uwc_cu_count();
 
+// go(r0, n) launches rows r0 .. r0 + n - 1 with a workgroup of `threads` per row. A launch holds fewer
+// than 2^32 threads (a larger grid is cut off without an error), so more rows than that go out in parts.
+template <class Go>
+static inline int uwc_launch_rows(const char* fn, int rows, unsigned threads, Go&& go) {
+  const long per = 0xFFFFFFFFu / threads;
+  for (long r0 = 0; r0 < rows; r0 += per) {
+    go(r0, (int)(rows - r0 < per ? rows - r0 : per));
+    if (int st = uwc_launch_status(fn)) return st;
+  }
+  return UWC_OK;
+}
+
 // ------------------------------------------------------------------ BLAKE3
 // The keyed one-block compression used for tile digests, noise words and tree nodes.
 // Restated from the BLAKE3 specification (the reference's CUDA version is

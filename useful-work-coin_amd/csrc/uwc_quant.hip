@@ -281,19 +281,24 @@ static int quant_rows(const char* fn, const T* x, int rows, int k, int bs, int q
   const bool ax = ((uintptr_t)x & 15) == 0;
   if (k % 16 == 0 && k <= 1024 * QD_MAX && bse <= 512 && ax && ((uintptr_t)q & 15) == 0 &&
       (k > 512 * QA_GMAX || (long)rows * ((k + 1023) / 1024) >= 2L * 4 * uwc_cu_count())) {
-    hipLaunchKernelGGL(quant_act_dgroup_kernel<T>, dim3((unsigned)rows), dim3(64 * ((k + 1023) / 1024)), 0, stream, x, k,
-                       lbs, qmax, q, scale);
-    return uwc_launch_status(fn);
+    const unsigned threads = 64 * ((k + 1023) / 1024);
+    return uwc_launch_rows(fn, rows, threads, [&](long r0, int n) {
+      hipLaunchKernelGGL(quant_act_dgroup_kernel<T>, dim3((unsigned)n), dim3(threads), 0, stream, x + r0 * k, k, lbs, qmax,
+                         q + r0 * k, scale + r0);
+    });
   }
   if (k % 8 == 0 && k <= 512 * QA_GMAX && bse <= 512 && ax && ((uintptr_t)q & 7) == 0) {
-    hipLaunchKernelGGL(quant_act_group_kernel<T>, dim3((unsigned)rows), dim3(64 * ((k + 511) / 512)), 0, stream, x, k, lbs,
-                       qmax, q, scale);
-    return uwc_launch_status(fn);
+    const unsigned threads = 64 * ((k + 511) / 512);
+    return uwc_launch_rows(fn, rows, threads, [&](long r0, int n) {
+      hipLaunchKernelGGL(quant_act_group_kernel<T>, dim3((unsigned)n), dim3(threads), 0, stream, x + r0 * k, k, lbs, qmax,
+                         q + r0 * k, scale + r0);
+    });
   }
   if (k % 512 == 0 && bse <= 512 && ax && ((uintptr_t)q & 7) == 0) {
-    hipLaunchKernelGGL(quant_act_wave_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, x, rows, k, lbs,
-                       qmax, q, scale);
-    return uwc_launch_status(fn);
+    return uwc_launch_rows(fn, rows, 256, [&](long r0, int n) {
+      hipLaunchKernelGGL(quant_act_wave_kernel<T>, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream, x + r0 * k, n, k,
+                         lbs, qmax, q + r0 * k, scale + r0);
+    });
   }
   const size_t smem = (size_t)k * 4;
   if (smem > 160 * 1024) return uwc_fail("%s: a row of k=%d floats exceeds LDS", fn, k);
@@ -301,8 +306,10 @@ static int quant_rows(const char* fn, const T* x, int rows, int k, int bs, int q
     hipError_t e = hipFuncSetAttribute((const void*)quant_act_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) return uwc_fail("%s: cannot raise LDS to %zu bytes: %s", fn, smem, hipGetErrorString(e));
   }
-  hipLaunchKernelGGL(quant_act_kernel<T>, dim3(rows), dim3(256), smem, stream, x, k, bs, qmax, q, scale);
-  return uwc_launch_status(fn);
+  return uwc_launch_rows(fn, rows, 256, [&](long r0, int n) {
+    hipLaunchKernelGGL(quant_act_kernel<T>, dim3((unsigned)n), dim3(256), smem, stream, x + r0 * k, k, bs, qmax, q + r0 * k,
+                       scale + r0);
+  });
 }
 
 extern "C" int uwc_quant_act_f32(const float* x, int rows, int k, int bs, int qmax, int8_t* q, float* scale,
