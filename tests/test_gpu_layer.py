@@ -570,17 +570,28 @@ def test_sha_row_roots_shapes(dev, rows, words):
         assert bytes(got_l[i]) == S.tagged_leaf(b"sout", (5 + i) % 7, want)
 
 
-@pytest.mark.parametrize("op,rows,k", [("quant", (1 << 26) + 3, 8), ("quant", (1 << 26) + 3, 16), ("quant", (1 << 24) + 3, 9)])
+@pytest.mark.parametrize("op,rows,k", [("quant", (1 << 26) + 3, 8), ("quant", (1 << 26) + 3, 16), ("quant", (1 << 24) + 3, 9),
+                                       ("swiglu", (1 << 24) + 3, 8), ("swiglu", (1 << 24) + 3, 9), ("rmsnorm", (1 << 26) + 3, 8),
+                                       ("rmsnorm", (1 << 24) + 3, 9), ("embed", (1 << 24) + 3, 4)])
 def test_row_kernels_past_one_launch(dev, op, rows, k):
     """More rows than one launch of a workgroup per row may hold (2^32 threads): every row as in calls
     over the halves, which fit."""
     from uwc_amd import detgpu
     g = torch.Generator(device=dev)
     g.manual_seed(k)
-    x = torch.randn((rows, k), device=dev, generator=g)
-    run = lambda a, b: detgpu.quant_act(x[a:b], k & -k)
-    q, s = run(0, rows)
-    h = rows // 2
+    if op == "swiglu":
+        x = torch.randint(-1 << 20, 1 << 20, (rows, 2 * k), dtype=torch.int32, device=dev, generator=g)
+        s3, sw = torch.rand(rows, device=dev, generator=g) * 1e-4, torch.rand(2 * k, device=dev, generator=g)
+        run = lambda a, b: detgpu.swiglu_quant(x[a:b], s3[a:b], sw, k & -k)
+    elif op == "embed":
+        x = torch.randint(0, 1000, (rows,), device=dev, generator=g)
+        table = torch.randn((1000, k), device=dev, generator=g)
+        run = lambda a, b: (detgpu.embed(table, x[a:b]),)
+    else:
+        x = torch.randn((rows, k), device=dev, generator=g)
+        w = torch.rand(k, device=dev, generator=g)
+        run = lambda a, b: detgpu.quant_act(x[a:b], k & -k) if op == "quant" else detgpu.rmsnorm_quant(x[a:b], w, 1e-6, k & -k)
+    whole, h = run(0, rows), rows // 2
     for a, b in ((0, h), (h, rows)):
-        qh, sh = run(a, b)
-        assert torch.equal(q[a:b], qh) and torch.equal(s[a:b].view(torch.int32), sh.view(torch.int32))
+        for w_, p in zip(whole, run(a, b)):
+            assert torch.equal(w_[a:b], p)

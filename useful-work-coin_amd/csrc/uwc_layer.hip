@@ -511,25 +511,26 @@ extern "C" int uwc_rmsnorm_quant_f32(const float* x, const float* w, int rows, i
   if (k % 8 == 0 && k <= 16384 && bse <= 512 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 &&
       ((uintptr_t)q & 7) == 0) {
     const int lbs = __builtin_ctz((unsigned)bse);
-#define RMSQ(G, W)                                                                                                 \
-  case G:                                                                                                          \
-    hipLaunchKernelGGL((k % (512 * W) ? rmsnorm_quant_regs_kernel<G, W, true> : rmsnorm_quant_regs_kernel<G, W, false>), \
-                       dim3(W > 1 ? (unsigned)rows : (unsigned)((rows + 3) / 4)), dim3(256), 0, stream, x, w, rows, k, \
-                       lbs, inv_d, eps, q, scale);                                                                 \
-    break;
+#define RMSQ(G, W)                                                                                                        \
+  case G:                                                                                                                 \
+    return uwc_launch_rows(fn, rows, 256, [&](long r0, int n) {                                                           \
+      hipLaunchKernelGGL((k % (512 * W) ? rmsnorm_quant_regs_kernel<G, W, true> : rmsnorm_quant_regs_kernel<G, W, false>), \
+                         dim3((unsigned)(W > 1 ? n : (n + 3) / 4)), dim3(256), 0, stream, x + r0 * k, w, n, k, lbs, inv_d,  \
+                         eps, q + r0 * k, scale + r0);                                                                    \
+    });
     if (k > 4096 || (k > 512 && rows < 4 * uwc_cu_count())) {
       switch ((k + 2047) / 2048) { RMSQ(1, 4) RMSQ(2, 4) RMSQ(3, 4) RMSQ(4, 4) RMSQ(5, 4) RMSQ(6, 4) RMSQ(7, 4) RMSQ(8, 4) }
     } else {
       switch ((k + 511) / 512) { RMSQ(1, 1) RMSQ(2, 1) RMSQ(3, 1) RMSQ(4, 1) RMSQ(5, 1) RMSQ(6, 1) RMSQ(7, 1) RMSQ(8, 1) }
     }
 #undef RMSQ
-    return uwc_launch_status(fn);
   }
   size_t smem;
   if ((st = row_lds(fn, (const void*)rmsnorm_kernel<true>, k, smem))) return st;
-  hipLaunchKernelGGL(rmsnorm_kernel<true>, dim3(rows), dim3(256), smem, stream, x, w, k, bs, inv_d, eps, q, scale,
-                     (float*)nullptr);
-  return uwc_launch_status(fn);
+  return uwc_launch_rows(fn, rows, 256, [&](long r0, int n) {
+    hipLaunchKernelGGL(rmsnorm_kernel<true>, dim3((unsigned)n), dim3(256), smem, stream, x + r0 * k, w, k, bs, inv_d, eps,
+                       q + r0 * k, scale + r0, (float*)nullptr);
+  });
 }
 
 extern "C" int uwc_rmsnorm_f32(const float* x, const float* w, int rows, int k, float inv_d, float eps, float* y,
@@ -540,9 +541,10 @@ extern "C" int uwc_rmsnorm_f32(const float* x, const float* w, int rows, int k, 
   size_t smem;
   int st = row_lds(fn, (const void*)rmsnorm_kernel<false>, k, smem);
   if (st) return st;
-  hipLaunchKernelGGL(rmsnorm_kernel<false>, dim3(rows), dim3(256), smem, stream, x, w, k, 0, inv_d, eps,
-                     (i8*)nullptr, (float*)nullptr, y);
-  return uwc_launch_status(fn);
+  return uwc_launch_rows(fn, rows, 256, [&](long r0, int n) {
+    hipLaunchKernelGGL(rmsnorm_kernel<false>, dim3((unsigned)n), dim3(256), smem, stream, x + r0 * k, w, k, 0, inv_d, eps,
+                       (i8*)nullptr, (float*)nullptr, y + r0 * k);
+  });
 }
 
 extern "C" int uwc_swiglu_quant(const void* acc, const float* s3, const float* sw, int rows, int I, int bs,
@@ -558,24 +560,22 @@ extern "C" int uwc_swiglu_quant(const void* acc, const float* s3, const float* s
       ((uintptr_t)q & 7) == 0) {
     const int lbs = __builtin_ctz((unsigned)bse);
     const i32* a = static_cast<const i32*>(acc);
-#define SWQ(G)                                                                                                \
-  case G:                                                                                                     \
-    hipLaunchKernelGGL(swiglu_quant_regs_kernel<G>, dim3((unsigned)rows), dim3(256), 0, stream, a, s3, sw, I, \
-                       lbs, q, scale);                                                                        \
-    break;
+#define SWQ(G)                                                                                                 \
+  case G:                                                                                                      \
+    return uwc_launch_rows(fn, rows, 256, [&](long r0, int n) {                                                \
+      hipLaunchKernelGGL(swiglu_quant_regs_kernel<G>, dim3((unsigned)n), dim3(256), 0, stream, a + r0 * 2 * I, \
+                         s3 + r0, sw, I, lbs, q + r0 * I, scale + r0);                                         \
+    });
     switch ((I + 2047) / 2048) { SWQ(1) SWQ(2) SWQ(3) SWQ(4) SWQ(5) SWQ(6) SWQ(7) SWQ(8) }
 #undef SWQ
-    return uwc_launch_status(fn);
   }
   size_t smem;
-  if (s3) {
-    if ((st = row_lds(fn, (const void*)swiglu_quant_kernel<false>, I, smem))) return st;
-    hipLaunchKernelGGL(swiglu_quant_kernel<false>, dim3(rows), dim3(256), smem, stream, acc, s3, sw, I, bs, q, scale);
-  } else {
-    if ((st = row_lds(fn, (const void*)swiglu_quant_kernel<true>, I, smem))) return st;
-    hipLaunchKernelGGL(swiglu_quant_kernel<true>, dim3(rows), dim3(256), smem, stream, acc, s3, sw, I, bs, q, scale);
-  }
-  return uwc_launch_status(fn);
+  const auto kern = s3 ? swiglu_quant_kernel<false> : swiglu_quant_kernel<true>;
+  if ((st = row_lds(fn, (const void*)kern, I, smem))) return st;
+  return uwc_launch_rows(fn, rows, 256, [&](long r0, int n) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(256), smem, stream, static_cast<const u32*>(acc) + r0 * 2 * I,
+                       s3 ? s3 + r0 : nullptr, sw, I, bs, q + r0 * I, scale + r0);
+  });
 }
 
 extern "C" int uwc_dequant_residual(const void* acc, const float* s, const float* sw, const float* x, int rows, int n,
@@ -599,8 +599,10 @@ extern "C" int uwc_embed_rows(const float* table, int64_t V, int D, const int64_
   const char* fn = "uwc_embed_rows";
   if (!table || !ids || !out || V <= 0 || D <= 0 || N < 0) return uwc_fail("%s: null or empty arguments", fn);
   if (N == 0) return UWC_OK;
-  hipLaunchKernelGGL(embed_kernel, dim3(N), dim3(256), 0, stream, table, (long)V, D, ids, N, out, bad);
-  return uwc_launch_status(fn);
+  return uwc_launch_rows(fn, N, 256, [&](long r0, int n) {
+    hipLaunchKernelGGL(embed_kernel, dim3((unsigned)n), dim3(256), 0, stream, table, (long)V, D, ids + r0, n, out + r0 * D,
+                       bad);
+  });
 }
 
 extern "C" int uwc_vt_tokens(int T) { return T <= 0 ? 0 : ((T + 63) / 64) * 64; }
