@@ -517,6 +517,15 @@ def test_quantizing_row_kernels_widths(dev, rows, k, bs):
     assert np.array_equal(q.cpu().numpy()[pick], rq) and np.array_equal(_u32(s)[pick], _u32(rs))
 
 
+@pytest.mark.parametrize("k,bs", [(256, 64), (264, 8), (512, 512), (1024, 256), (1032, 8), (1536, 512), (1544, 8), (2560, 512),
+                                  (3584, 128), (3592, 8), (4096, 64)])
+@pytest.mark.parametrize("rows", [256, 257, 513, 769, 1025])
+def test_quantizing_row_kernels_dispatch_edges(dev, rows, k, bs):
+    """The same on both sides of every line between their forms: widths around whole groups and row
+    counts around one, two, three and four rows per CU."""
+    test_quantizing_row_kernels_widths(dev, rows, k, bs)
+
+
 @pytest.mark.parametrize("B,T,H,Hkv,hd,I,D,arch", [(1, 1, 2, 1, 32, 128, 64, 0), (2, 70, 4, 2, 64, 384, 256, 1),
                                                     (1, 200, 4, 4, 128, 640, 512, 0), (3, 64, 2, 2, 32, 512, 128, 0)])
 def test_layer_call_equals_ops(dev, B, T, H, Hkv, hd, I, D, arch, monkeypatch):

@@ -40,18 +40,16 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const float* __restrict__ 
   }
 }
 
-// A row in the registers of W waves (W = 1: a wave has its row to itself; W = 4: the workgroup's four
-// waves share one), G 512-element groups per wave: wave w of the row holds groups w, w + W, ..., lane
-// L elements 8 L .. 8 L + 7 of each (the layout of fwht512_rows). k % 8 == 0: lanes past the row's end
+// A row in the registers of W waves (W = 1: a wave has its row to itself; W > 1: the workgroup's waves
+// share one), G 512-element groups per wave: wave w of the row holds groups w, w + W, ..., lane L
+// elements 8 L .. 8 L + 7 of each (the layout of fwht512_rows). k % 8 == 0: lanes past the row's end
 // hold zeros and neither load nor store (bs divides k, so the transform keeps them zero).
 // TAIL: the row has such lanes (without them every test of the row's end is left out: 4% of a
 // 4096 x 2048 rmsnorm_quant).
 // One wave per row needs no LDS and no barrier, and the work that does not grow with the row runs
-// once; four waves per row finish it sooner and hold a quarter of the registers each. rmsnorm_quant
-// (k = 2048, us): one wave 5.0 / 5.3 / 7.6 / 9.4 / 24.0 at 200 / 600 / 1200 / 2000 / 8192 rows, four
-// 3.9 / 5.2 / 7.4 / 10.8 / 24.5, so four below four rows per CU and for rows one wave cannot hold.
-// swiglu_quant, whose work per element is several times that, is faster on four at every size (I =
-// 6144: 18.9 -> 7.2 at 200 rows, 36.9 -> 29.2 at 2000, 124 -> 107 at 8192).
+// once; more waves per row finish it sooner and hold a part of the registers each. Where the line
+// lies for rmsnorm_quant and for swiglu_quant, whose work per element is several times that, stands at
+// their dispatch.
 struct RowRed {
   float f[2][4];
   long long l[4];
@@ -64,7 +62,9 @@ __device__ __forceinline__ float row_max(float v, RowRed& red, int slot) {
   if constexpr (W > 1) {
     if ((threadIdx.x & 63) == 0) red.f[slot][threadIdx.x >> 6] = v;
     __syncthreads();
-    v = fmaxf(fmaxf(red.f[slot][0], red.f[slot][1]), fmaxf(red.f[slot][2], red.f[slot][3]));
+    v = red.f[slot][0];
+#pragma unroll
+    for (int i = 1; i < W; i++) v = fmaxf(v, red.f[slot][i]);
   }
   return v;
 }
@@ -159,26 +159,28 @@ __global__ void __launch_bounds__(256) rmsnorm_quant_regs_kernel(const float* __
 }
 
 // ------------------------------------------------------------------ swiglu + quant_act
-// swiglu_quant from int32 gate | up rows held in the registers of four waves (I <= 2048 G, bs <=
-// 512): element i = fmul(silu(deq(g_i)), deq(u_i)) as in the LDS row kernel below, then
-// quant_row_regs. VALU-bound (det_exp and the division: about 60 instructions an element) where the
-// LDS form waited on its nine passes and barriers: I = 14336 at 2000 rows 169 -> 70 us. The test of
-// the row's end stays in whole rows too: without it the compiler loads every group before the first
+// swiglu_quant from int32 gate | up rows held in the registers of W waves (I <= 512 W G, bs <= 512):
+// element i = fmul(silu(deq(g_i)), deq(u_i)) as in the LDS row kernel below, then quant_row_regs.
+// VALU-bound (det_exp and the division: about 60 instructions an element) where the LDS form waited on
+// its nine passes and barriers: I = 14336 at 2000 rows 169 -> 70 us. The test of the row's end stays in
+// whole rows of several groups per wave too: without it the compiler loads every group before the first
 // is worked on, and the registers cost more than the tests (I = 6144 at 8192 rows 107 -> 113 us).
-template <int G>
+template <int G, int W, bool TAIL>
 __global__ void __launch_bounds__(256) swiglu_quant_regs_kernel(const i32* __restrict__ acc, const float* __restrict__ s3,
-                                                                const float* __restrict__ sw, int I, int lbs,
+                                                                const float* __restrict__ sw, int rows, int row_I, int lbs,
                                                                 i8* __restrict__ q, float* __restrict__ scale) {
+  const int I = TAIL ? row_I : 512 * G * W;
   __shared__ RowRed red;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long r = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = W > 1 ? threadIdx.x >> 6 : 0;
+  const long r = W > 1 ? (long)blockIdx.x : (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= rows) return;  // W = 1: whole waves, and no barriers below; W > 1: never
   const i32* ar = acc + r * 2L * I;
   const float sx = s3[r];
   float y[G][8];
 #pragma unroll
   for (int g = 0; g < G; g++) {
-    const int at = (4 * g + wave) * 512 + lane * 8;
-    if (at < I) {
+    const int at = (W * g + wave) * 512 + lane * 8;
+    if (!TAIL || at < I) {
       const v4i g0 = *reinterpret_cast<const v4i*>(ar + at), g1 = *reinterpret_cast<const v4i*>(ar + at + 4);
       const v4i u0 = *reinterpret_cast<const v4i*>(ar + I + at), u1 = *reinterpret_cast<const v4i*>(ar + I + at + 4);
       const float4 wg0 = *reinterpret_cast<const float4*>(sw + at), wg1 = *reinterpret_cast<const float4*>(sw + at + 4);
@@ -194,7 +196,7 @@ __global__ void __launch_bounds__(256) swiglu_quant_regs_kernel(const i32* __res
       for (int j = 0; j < 8; j++) y[g][j] = 0.0f;
     }
   }
-  quant_row_regs<G, 4, true>(y, lane, wave, I, lbs, q + r * (long)I, scale + r, red);
+  quant_row_regs<G, W, TAIL>(y, lane, wave, I, lbs, q + r * (long)I, scale + r, red);
 }
 
 // acc: rows x 2I (gate | up), int32 accumulators dequantized with s3[row], sw[col], or with FP
@@ -518,6 +520,8 @@ extern "C" int uwc_rmsnorm_quant_f32(const float* x, const float* w, int rows, i
                          dim3((unsigned)(W > 1 ? n : (n + 3) / 4)), dim3(256), 0, stream, x + r0 * k, w, n, k, lbs, inv_d,  \
                          eps, q + r0 * k, scale + r0);                                                                    \
     });
+    // four waves per row below four rows per CU and for rows one wave cannot hold (k = 2048, us): one wave 5.0 /
+    // 5.3 / 7.6 / 9.4 / 24.0 at 200 / 600 / 1200 / 2000 / 8192 rows, four 3.9 / 5.2 / 7.4 / 10.8 / 24.5
     if (k > 4096 || (k > 512 && rows < 4 * uwc_cu_count())) {
       switch ((k + 2047) / 2048) { RMSQ(1, 4) RMSQ(2, 4) RMSQ(3, 4) RMSQ(4, 4) RMSQ(5, 4) RMSQ(6, 4) RMSQ(7, 4) RMSQ(8, 4) }
     } else {
@@ -556,17 +560,39 @@ extern "C" int uwc_swiglu_quant(const void* acc, const float* s3, const float* s
   if (st) return st;
   if (rows == 0) return UWC_OK;
   const int bse = bs > 1 ? bs : 1;
-  if (s3 && I % 8 == 0 && I <= 16384 && bse <= 512 && ((uintptr_t)acc & 15) == 0 && ((uintptr_t)sw & 15) == 0 &&
+  if (s3 && I % 8 == 0 && I > 256 && I <= 16384 && bse <= 512 && ((uintptr_t)acc & 15) == 0 && ((uintptr_t)sw & 15) == 0 &&
       ((uintptr_t)q & 7) == 0) {
     const int lbs = __builtin_ctz((unsigned)bse);
     const i32* a = static_cast<const i32*>(acc);
-#define SWQ(G)                                                                                                 \
-  case G:                                                                                                      \
-    return uwc_launch_rows(fn, rows, 256, [&](long r0, int n) {                                                \
-      hipLaunchKernelGGL(swiglu_quant_regs_kernel<G>, dim3((unsigned)n), dim3(256), 0, stream, a + r0 * 2 * I, \
-                         s3 + r0, sw, I, lbs, q + r0 * I, scale + r0);                                         \
-    });
-    switch ((I + 2047) / 2048) { SWQ(1) SWQ(2) SWQ(3) SWQ(4) SWQ(5) SWQ(6) SWQ(7) SWQ(8) }
+#define SWQ(G, W, TAIL)                                                                                            \
+  return uwc_launch_rows(fn, rows, 256, [&](long r0, int n) {                                                      \
+    hipLaunchKernelGGL((swiglu_quant_regs_kernel<G, W, TAIL>), dim3((unsigned)(W > 1 ? n : (n + 3) / 4)),          \
+                       dim3(W > 1 ? 64 * W : 256), 0, stream, a + r0 * 2 * I, s3 + r0, sw, n, I, lbs, q + r0 * I, \
+                       scale + r0);                                                                                \
+  })
+    // a wave per 512-element group up to four (us against four waves whatever the width: I = 512 at 1000 /
+    // 8192 / 32768 rows 4.8 -> 3.9 / 18.7 -> 11.0 / 63 -> 32; 1024 at 700 rows 4.9 -> 4.7; 1536 at 1200 rows
+    // 6.9 -> 6.5), but one wave with two groups for many rows of 1024 (8192 rows 23.1 -> 18.6). Wider rows: four
+    // beat one at every row count (I = 6144: 18.9 -> 7.2 at 200, 36.9 -> 29.2 at 2000, 124 -> 107 at 8192).
+    // Rows of at most 256 elements keep the LDS form, a thread per element (256 x 64 3.8 -> 3.5, 8192 x 64 15 -> 10).
+    if (I == 512) SWQ(1, 1, false);
+    if (I == 1024 && rows > 4 * uwc_cu_count()) SWQ(2, 1, false);
+    if (I == 1536) SWQ(1, 3, false);
+    switch ((I + 511) / 512) {
+      case 1: SWQ(1, 1, true);
+      case 2: SWQ(1, 2, true);
+      case 3: SWQ(1, 3, true);
+    }
+    switch ((I + 2047) / 2048) {
+      case 1: SWQ(1, 4, true);
+      case 2: SWQ(2, 4, true);
+      case 3: SWQ(3, 4, true);
+      case 4: SWQ(4, 4, true);
+      case 5: SWQ(5, 4, true);
+      case 6: SWQ(6, 4, true);
+      case 7: SWQ(7, 4, true);
+      case 8: SWQ(8, 4, true);
+    }
 #undef SWQ
   }
   size_t smem;
