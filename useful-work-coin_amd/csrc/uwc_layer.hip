@@ -115,8 +115,9 @@ __device__ __forceinline__ void quant_row_regs(float (&y)[G][8], int lane, int w
 // us of traffic; 25 so).
 template <int G, int W, bool TAIL>
 __global__ void __launch_bounds__(256) rmsnorm_quant_regs_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                                 int rows, int k, int lbs, float inv_d, float eps,
+                                                                 int rows, int row_k, int lbs, float inv_d, float eps,
                                                                  i8* __restrict__ q, float* __restrict__ scale) {
+  const int k = TAIL || W > 1 ? row_k : 512 * G;
   __shared__ RowRed red;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wv = W > 1 ? wave : 0;
   const long r = W > 1 ? (long)blockIdx.x : (long)blockIdx.x * 4 + wave;
@@ -520,9 +521,14 @@ extern "C" int uwc_rmsnorm_quant_f32(const float* x, const float* w, int rows, i
                          dim3((unsigned)(W > 1 ? n : (n + 3) / 4)), dim3(256), 0, stream, x + r0 * k, w, n, k, lbs, inv_d,  \
                          eps, q + r0 * k, scale + r0);                                                                    \
     });
-    // four waves per row below four rows per CU and for rows one wave cannot hold (k = 2048, us): one wave 5.0 /
-    // 5.3 / 7.6 / 9.4 / 24.0 at 200 / 600 / 1200 / 2000 / 8192 rows, four 3.9 / 5.2 / 7.4 / 10.8 / 24.5
-    if (k > 4096 || (k > 512 && rows < 4 * uwc_cu_count())) {
+    // four waves per row up to per_cu rows per CU, one beyond (us, one wave / four: k = 2048 5.5 / 4.0 at
+    // 200 rows, 5.7 / 5.4 at 600, 5.7 / 6.1 at 777, 7.2 / 7.4 at 1200, 22 / 28 at 8192; k = 4096 9.1 / 8.1 at
+    // 1000). One wave has no tail tests in whole rows and four leave some of theirs without a group at 1536
+    // and 2560 (1536: 4.8 / 5.3 at 600 rows), so whole rows turn earlier there and take one wave throughout
+    // up to 1024 (4.0 / 6.0 at 1000 rows); 768: 4.2 / 3.9 at 200 rows, 4.3 / 5.0 at 600. Past 4096 one wave
+    // cannot hold a row.
+    const int per_cu = k > 3584 ? 4 : k <= 1024 ? k > 512 && k % 512 : k % 512 == 0 && k % 2048 && k < 3072 ? 2 : 3;
+    if (k > 4096 || rows <= per_cu * uwc_cu_count()) {
       switch ((k + 2047) / 2048) { RMSQ(1, 4) RMSQ(2, 4) RMSQ(3, 4) RMSQ(4, 4) RMSQ(5, 4) RMSQ(6, 4) RMSQ(7, 4) RMSQ(8, 4) }
     } else {
       switch ((k + 511) / 512) { RMSQ(1, 1) RMSQ(2, 1) RMSQ(3, 1) RMSQ(4, 1) RMSQ(5, 1) RMSQ(6, 1) RMSQ(7, 1) RMSQ(8, 1) }
