@@ -517,6 +517,12 @@ def test_quantizing_row_kernels_widths(dev, rows, k, bs):
     assert np.array_equal(q.cpu().numpy()[pick], rq) and np.array_equal(_u32(s)[pick], _u32(rs))
 
 
+@pytest.mark.parametrize("rows,words", [(63, 256), (65, 256), (64, 300), (130, 1024), (4097, 300), (16385, 300)])
+def test_sha_row_roots_workgroup_edges(dev, rows, words):
+    """Row trees just under, at and past the 64 rows of a workgroup, at one, two and four blocks per row."""
+    test_sha_row_roots_shapes(dev, rows, words)
+
+
 @pytest.mark.parametrize("k,bs", [(256, 64), (264, 8), (512, 512), (1024, 256), (1032, 8), (1536, 512), (1544, 8), (2560, 512),
                                   (3584, 128), (3592, 8), (4096, 64)])
 @pytest.mark.parametrize("rows", [256, 257, 513, 769, 1025])

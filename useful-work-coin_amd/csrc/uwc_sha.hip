@@ -221,10 +221,11 @@ __global__ void sha_row_leaf_kernel(u32* __restrict__ leaves, long nrows, int nb
 // block leaves in LDS, each level's parents computed in parallel over all of the rows into a second
 // buffer (an odd last node moves up), then the tagged leaves, one thread per row. A thread per row
 // would run its 2 (nblk - 1) compressions one after another. per nblk is about 512 leaves, so that
-// the first level fills the workgroup. The levels' latency (two compressions each, about 3 us for a
-// wave alone on its SIMD) bounds it. 32,768 rows of 8 blocks: 73 us with a quad of lanes per row and
-// 16 rows per wave, 34 so; rows of 594 blocks, one per workgroup, 102 at 300 rows (23 compressions
-// one after another are 70).
+// the first level fills the workgroup, of at most 64 rows: with 256 a handful of workgroups loads all the
+// leaves of short rows (4096 rows of 2 blocks 14.1 -> 9.9 us, 1000 of one 6.4 -> 4.8). The levels' latency
+// (two compressions each, about 3 us for a wave alone on its SIMD) bounds it. 32,768 rows of 8 blocks: 73
+// us with a quad of lanes per row and 16 rows per wave, 34 so; rows of 594 blocks, one per workgroup, 102
+// at 300 rows (23 compressions one after another are 70).
 #define SHA_ROWTREE_MAXBLK 1024
 #define SHA_ROWTREE_LEAVES 512
 __global__ void __launch_bounds__(256) sha_row_tree_kernel(const u32* __restrict__ leaves, long nrows, int nblk, int per,
@@ -356,11 +357,12 @@ extern "C" int uwc_sha_row_leaves(const uint32_t* rows, int64_t nrows, int row_w
     return uwc_fail("%s: scratch has %lld words, needs %lld", fn, (long long)scratch_words, (long long)(nrows * nblk * 8));
   const long nt = nrows * nblk;
   // four waves per workgroup, one per SIMD: with two, a CU's workgroups share two of its SIMDs (8192
-  // rows of 2048 words 90 -> 56 us, 300 of 151,936 190 -> 149). While the waves are no more than one
-  // or two per CU, workgroups of one or two spread them over the CUs (186 and 372 waves, 20 and 40 rows
-  // of 151,936: 57.2 -> 55.7 us; logits of 20 rows with their roots 198 -> 196, of 6 rows 186 -> 184)
+  // rows of 2048 words 96 -> 61 us, 300 of 151,936 190 -> 149). While the waves are no more than two per
+  // CU, workgroups of two spread them over the CUs (20 and 40 rows of 151,936 words 57.2 -> 55.1 us).
+  // Workgroups of one wave do so no better and are slower where lanes run out or end early (4096 rows of
+  // 300 words 51 -> 64 us, 200 of 256 50 -> 56, one of 151,936 51 -> 57).
   const long waves = (nt + 63) / 64, cus = uwc_cu_count();
-  const int threads = waves <= cus ? 64 : waves <= 2 * cus ? 128 : 256;
+  const int threads = waves <= 2 * cus ? 128 : 256;
   const dim3 grid((unsigned)((nt + threads - 1) / threads));
   if (row_words % 4 == 0 && ((uintptr_t)rows & 15) == 0)
     hipLaunchKernelGGL(sha_block_leaves_kernel<true>, grid, dim3(threads), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
@@ -368,7 +370,7 @@ extern "C" int uwc_sha_row_leaves(const uint32_t* rows, int64_t nrows, int row_w
     hipLaunchKernelGGL(sha_block_leaves_kernel<false>, grid, dim3(threads), 0, stream, rows, (long)nrows, row_words, nblk, scratch);
   int st = uwc_launch_status("sha_block_leaves");
   if (st) return st;
-  const int per = nblk >= SHA_ROWTREE_LEAVES ? 1 : SHA_ROWTREE_LEAVES / nblk < 256 ? SHA_ROWTREE_LEAVES / nblk : 256;
+  const int per = nblk >= SHA_ROWTREE_LEAVES ? 1 : SHA_ROWTREE_LEAVES / nblk < 64 ? SHA_ROWTREE_LEAVES / nblk : 64;
   if (nblk <= SHA_ROWTREE_MAXBLK && (nrows + per - 1) / per <= 0x7FFFFFFFL)
     hipLaunchKernelGGL(sha_row_tree_kernel, dim3((unsigned)((nrows + per - 1) / per)), dim3(256),
                        (size_t)per * (nblk + (nblk + 1) / 2) * 32, stream, scratch, (long)nrows, nblk, per, tag,
