@@ -94,6 +94,18 @@ int uwc_noisy_gemm_many(int count, const int8_t* const* A, const int8_t* B, int 
                         const float* a_scale, const float* b_scale, void* const* out, int out_mode, int flags,
                         uint32_t* const* tile_dump, hipStream_t stream);
 
+/* Which kernel a plain GEMM of this shape runs on, its operands and outputs 16-byte aligned (host side,
+ * no GPU work): 0 .. 8, a form of the plain kernels (128 x 128 tiles with a 4-step or a 2-step ring, 64 x
+ * 128, 64 x 64 on two or four waves, 64 x 32, 32 x 32, 16 x 32, 16 x 16), or one of UWC_ROUTE_*. second:
+ * 1 with a residual (uwc_igemm_dequant_residual_f32, UWC_OUT_F32), 2 with the dequantized rows beside the
+ * int32 ones (uwc_igemm_i32_dequant_f32, UWC_OUT_I32), else 0. cus: a CU count, 0 the device's. */
+#define UWC_ROUTE_LARGE 16          /* 256 x 256 tiles */
+#define UWC_ROUTE_LARGE_COLUMNS 17  /* 256 x 256 tiles, then the last n % 256 columns */
+#define UWC_ROUTE_SKINNY 18         /* m <= 64, X in LDS */
+#define UWC_ROUTE_SKINNY_STREAM 19  /* m <= 64, X larger than LDS */
+#define UWC_ROUTE_STAGED 20         /* register-staged 128 x 128 tiles */
+int uwc_plain_gemm_route(int m, int n, int k, int out_mode, int second, int cus);
+
 /* Exact int32 C = A * B^T for any m, n (k % 64 == 0).
  * Replaces DetLinear.int_gemm's GPU path (torch._int_mm / MinedWeight.forward OUT_I32):
  * runtime/detrt/qwen3.py:106-119. */

@@ -331,8 +331,10 @@ bool uwc_plain_fits(int cfg, int m, int n, int k, int ldc, const void* out, int 
 int uwc_gemm_plain(int cfg, const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
                    const float* b_scale, void* out, int out_mode, int ldc, hipStream_t stream);
 
-bool uwc_plain_any_fits(int n, int k, int ldc, const void* out, int out_mode, const float* b_scale, const float* res,
-                        const float* out2);
+bool uwc_plain_any_fits(int m, int n, int k, int ldc, const void* out, int out_mode, const float* b_scale,
+                        const float* res, const float* out2);
+int uwc_plain_form(int m, int n, int k, int out_mode, int out_bytes, int cus);
+bool uwc_skinny_resident(int m, int k);
 int uwc_gemm_plain_any(const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
                        const float* b_scale, const float* res, void* out, float* out2, int out_mode, int ldc,
                        hipStream_t stream);
@@ -348,6 +350,28 @@ static void launch_out(int out_mode, dim3 grid, hipStream_t s, const GemmParams&
 }
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+
+// Whether the 256 x 256 kernel takes all of an m x n x k GEMM. Its DMA adds 32-bit lane offsets (255 k +
+// 112) and its row stores 32-bit offsets (31 ldc elements of 4 bytes): k and the output row stride stay
+// below 2^24.
+static bool takes256(int m, int n, int k) {
+  return m % 256 == 0 && n % 256 == 0 && k % 128 == 0 && k <= (1 << 24) && n <= (1 << 24);
+}
+
+// How much of a plain GEMM runs on 256 x 256 tiles: all of it while they keep the CUs busy (at least one
+// tile per CU and the last round of tiles at least 90% full: 2048 x 12288 gives 384 tiles on 256 CUs, a
+// half-empty second round, and runs faster on the plain kernels), or, where n is not a multiple of 256
+// (e.g. a vocabulary of 151936), the columns before the last multiple. vec_out: the 256 x 256 epilogue
+// writes 16-byte (8-byte for bf16) row segments, so rows must start aligned.
+enum { LARGE_NONE, LARGE_WHOLE, LARGE_COLUMNS };
+static int large_tiles(int m, int n, int k, bool vec_out, int cus) {
+  const int n256 = n / 256 * 256;
+  if (!vec_out || n > (1 << 24) || !takes256(m, n256, k)) return LARGE_NONE;
+  const long t = (long)(m / 256) * (n256 / 256), rounds = (t + cus - 1) / cus;
+  if (t < cus) return LARGE_NONE;
+  if (n256 < n) return LARGE_COLUMNS;
+  return t * 10 >= rounds * cus * 9 ? LARGE_WHOLE : LARGE_NONE;
+}
 
 // The argument checks of uwc_noisy_gemm (status 0 or UWC_EINVAL with the message set).
 static int gemm_check(const int8_t* A, const int8_t* B, int m, int n, int k, int r, const int8_t* corrA,
@@ -402,34 +426,27 @@ extern "C" int uwc_noisy_gemm(const int8_t* A, const int8_t* B, int m, int n, in
   if (flags & FLAG_PLAIN)  // checked: a plain GEMM the forced configuration takes
     return uwc_gemm_plain((flags & FLAG_PLAIN_MASK) >> FLAG_PLAIN_SHIFT, A, B, m, n, k, a_scale, b_scale, out,
                           out_mode, n, stream);
-  // 256 x 256 tiles when hashing (one tiling per nonce shape), or for a plain GEMM when they keep
-  // the CUs busy: at least one tile per CU and the last round of tiles at least 90% full (2048 x
-  // 12288 gives 384 tiles on 256 CUs, a half-empty second round, and runs faster on the plain
-  // kernel's 128 x 128 tiles).
-  const int cus = uwc_cu_count();
-  const long t256 = (long)(m / 256) * (n / 256), rounds256 = (t256 + cus - 1) / cus;
-  const bool fills = t256 >= cus && t256 * 10 >= rounds256 * cus * 9;
-  // the 256 x 256 DMA adds 32-bit lane offsets (255 k + 112) and its row stores 32-bit offsets
-  // (31 ldc elements of 4 bytes): k and the output row stride stay below 2^24
-  const bool k256 = k % 128 == 0 && k <= (1 << 24) && n <= (1 << 24);
-  // the 256 x 256 epilogue writes 16-byte (8-byte for bf16) row segments: rows must start aligned
+  const bool tile128 = flags & FLAG_TILE128;
   const bool vec_out = out_mode == OUT_NONE || (aligned16(out) && n % 4 == 0);
-  if (m % 256 == 0 && n % 256 == 0 && k256 && vec_out && !(flags & FLAG_TILE128) && (!plain || fills))
+  // 256 x 256 tiles when hashing (one tiling per nonce shape), or for as much of a plain GEMM as
+  // large_tiles says
+  int large = LARGE_NONE;
+  if (!tile128)
+    large = plain ? large_tiles(m, n, k, vec_out, uwc_cu_count()) : vec_out && takes256(m, n, k) ? LARGE_WHOLE : LARGE_NONE;
+  if (large == LARGE_WHOLE)
     return uwc_noisy_gemm256(A, B, m, n, k, r, corrA, corrB, maxabs, lmax, key, target, wins, max_wins, a_scale,
-                             b_scale, out, out_mode, flags & ~FLAG_TILE128, tile_dump, n, stream);
-  // A plain GEMM whose n is not a multiple of 256 (e.g. a vocabulary of 151936) but whose 256 x 256
-  // tiles would fill the CUs: columns [0, n256) on 256 x 256 tiles, the last n - n256 on 128 x 128
-  // tiles writing into the same rows (integer sums: the split cannot change a value).
-  const int n256 = n / 256 * 256;
-  if (plain && m % 256 == 0 && k256 && vec_out && n256 > 0 && n256 < n && !(flags & FLAG_TILE128) &&
-      (long)(m / 256) * (n256 / 256) >= 256) {
+                             b_scale, out, out_mode, flags, tile_dump, n, stream);
+  // columns [0, n256) on 256 x 256 tiles, the last n - n256 on smaller ones writing into the same rows
+  // (integer sums: the split cannot change a value)
+  if (large == LARGE_COLUMNS) {
+    const int n256 = n / 256 * 256;
     const int st = uwc_noisy_gemm256(A, B, m, n256, k, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, 0,
                                      a_scale, b_scale, out, out_mode, 0, nullptr, n, stream);
     if (st || out_mode == OUT_NONE) return st;
     const size_t es = out_mode == OUT_BF16 ? 2 : 4;
     const float* sw_tail = b_scale ? b_scale + n256 : nullptr;
     void* out_tail = static_cast<char*>(out) + n256 * es;
-    if (uwc_plain_any_fits(n - n256, k, n, out_tail, out_mode, sw_tail, nullptr, nullptr))
+    if (uwc_plain_any_fits(m, n - n256, k, n, out_tail, out_mode, sw_tail, nullptr, nullptr))
       return uwc_gemm_plain_any(A, B + (long)n256 * k, m, n - n256, k, a_scale, sw_tail, nullptr, out_tail, nullptr,
                                 out_mode, n, stream);
     GemmParams q{A, B + (long)n256 * k, m, n - n256, k, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, 0,
@@ -440,8 +457,8 @@ extern "C" int uwc_noisy_gemm(const int8_t* A, const int8_t* B, int m, int n, in
   }
   // Every other plain GEMM with k % 128 == 0 and whole 16-byte output pieces: the plain kernels, on
   // the form their own rule picks. Without those, small m goes to the skinny kernels.
-  if (plain && !(flags & FLAG_TILE128)) {
-    if (uwc_plain_any_fits(n, k, n, out, out_mode, b_scale, nullptr, nullptr))
+  if (plain && !tile128) {
+    if (uwc_plain_any_fits(m, n, k, n, out, out_mode, b_scale, nullptr, nullptr))
       return uwc_gemm_plain_any(A, B, m, n, k, a_scale, b_scale, nullptr, out, nullptr, out_mode, n, stream);
     if (m <= 64 && out_mode != OUT_NONE)
       return uwc_skinny_gemm(A, B, m, n, k, a_scale, b_scale, out, out_mode, stream);
@@ -481,27 +498,13 @@ extern "C" int uwc_igemm_dequant_residual_f32(const int8_t* A, const int8_t* B, 
     return st;
   const uintptr_t xa = (uintptr_t)x, ya = (uintptr_t)Y, bytes = (uintptr_t)m * (uintptr_t)n * 4;
   if (xa < ya + bytes && ya < xa + bytes) return uwc_fail("%s: Y overlaps x", fn);
-  // the shapes uwc_noisy_gemm puts on 256 x 256 tiles with one workgroup per tile (at least one
-  // tile per CU, the last round at least 90% full); their epilogue adds the residual
-  const int cus = uwc_cu_count();
-  const long t256 = (long)(m / 256) * (n / 256), rounds256 = (t256 + cus - 1) / cus;
-  const bool fills = t256 >= cus && t256 * 10 >= rounds256 * cus * 9;
-  const bool k256 = k % 128 == 0 && k <= (1 << 24) && n <= (1 << 24);
-  if (m % 256 == 0 && n % 256 == 0 && k256 && fills && aligned16(Y) && aligned16(x) && n % 4 == 0)
+  if (large_tiles(m, n, k, aligned16(Y) && aligned16(x) && n % 4 == 0, uwc_cu_count()) == LARGE_WHOLE)
     return uwc_gemm256_residual(A, B, m, n, k, sx, sw, x, Y, stream);
-  if (uwc_plain_any_fits(n, k, n, Y, OUT_F32, sw, x, nullptr))
+  if (uwc_plain_any_fits(m, n, k, n, Y, OUT_F32, sw, x, nullptr))
     return uwc_gemm_plain_any(A, B, m, n, k, sx, sw, x, Y, nullptr, OUT_F32, n, stream);
   // elsewhere: the dequantized product, then Y = fadd(x, Y) in place (each element read, then written)
   if (int st = uwc_igemm_dequant_f32(A, B, m, n, k, sx, sw, Y, stream)) return st;
   return uwc_dequant_residual(Y, nullptr, nullptr, x, m, n, Y, stream);
-}
-
-// 256 x 256 tiles over the first n / 256 * 256 columns where they fill the CUs (uwc_noisy_gemm above)
-static bool takes_large_tiles(int m, int n, int k) {
-  const int cus = uwc_cu_count();
-  const long t256 = (long)(m / 256) * (n / 256), rounds256 = (t256 + cus - 1) / cus;
-  const bool fills = n % 256 ? t256 >= 256 : t256 >= cus && t256 * 10 >= rounds256 * cus * 9;
-  return m % 256 == 0 && k % 128 == 0 && k <= (1 << 24) && n <= (1 << 24) && fills;
 }
 
 extern "C" int uwc_igemm_i32_dequant_f32(const int8_t* A, const int8_t* B, int m, int n, int k, const float* sx,
@@ -511,10 +514,25 @@ extern "C" int uwc_igemm_i32_dequant_f32(const int8_t* A, const int8_t* B, int m
   if (int st = gemm_check(A, B, m, n, k, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, 0, sx, sw, Y,
                           OUT_F32, 0))
     return st;
-  if (!takes_large_tiles(m, n, k) && uwc_plain_any_fits(n, k, n, C, OUT_I32, sw, nullptr, Y))
+  if (large_tiles(m, n, k, aligned16(C) && n % 4 == 0, uwc_cu_count()) == LARGE_NONE &&
+      uwc_plain_any_fits(m, n, k, n, C, OUT_I32, sw, nullptr, Y))
     return uwc_gemm_plain_any(A, B, m, n, k, sx, sw, nullptr, C, Y, OUT_I32, n, stream);
   if (int st = uwc_igemm_i32(A, B, m, n, k, C, stream)) return st;
   return uwc_dequant_f32(C, sx, sw, m, n, Y, stream);
+}
+
+extern "C" int uwc_plain_gemm_route(int m, int n, int k, int out_mode, int second, int cus) {
+  if (m <= 0 || n <= 0 || k <= 0 || k % G_BK || out_mode < OUT_NONE || out_mode > OUT_F32 || second < 0 || second > 2 ||
+      (second == 1 && out_mode != OUT_F32) || (second == 2 && out_mode != OUT_I32) || cus < 0)
+    return uwc_fail("uwc_plain_gemm_route: m=%d n=%d k=%d out_mode=%d second=%d cus=%d", m, n, k, out_mode, second, cus);
+  if (cus == 0) cus = uwc_cu_count();
+  const int large = large_tiles(m, n, k, out_mode == OUT_NONE || n % 4 == 0, cus);
+  if (large == LARGE_WHOLE) return UWC_ROUTE_LARGE;
+  if (large == LARGE_COLUMNS && second != 1) return UWC_ROUTE_LARGE_COLUMNS;
+  if (uwc_plain_any_fits(m, n, k, n, nullptr, out_mode, nullptr, nullptr, nullptr))
+    return uwc_plain_form(m, n, k, out_mode, second ? 8 : out_mode == OUT_NONE ? 0 : out_mode == OUT_BF16 ? 2 : 4, cus);
+  if (m <= 64 && out_mode != OUT_NONE) return uwc_skinny_resident(m, k) ? UWC_ROUTE_SKINNY : UWC_ROUTE_SKINNY_STREAM;
+  return UWC_ROUTE_STAGED;
 }
 
 int uwc_noisy_gemm256_many(int count, const int8_t* const* A, const int8_t* B, int m, int n, int k, int r,
@@ -534,8 +552,7 @@ extern "C" int uwc_noisy_gemm_many(int count, const int8_t* const* A, const int8
   const bool hash = flags & FLAG_HASH, denoise = flags & FLAG_DENOISE;
   if ((hash && !key) || (denoise && (!corrA || !corrB || !maxabs)))
     return uwc_fail("uwc_noisy_gemm_many: the flags need key / corrA, corrB, maxabs arrays");
-  bool split = count >= 2 && hash && denoise && out_mode == OUT_I32 && !(flags & FLAG_TILE128) && m % 256 == 0 &&
-               n % 256 == 0 && k % 128 == 0 && k <= (1 << 24) && n <= (1 << 24);
+  bool split = count >= 2 && hash && denoise && out_mode == OUT_I32 && !(flags & FLAG_TILE128) && takes256(m, n, k);
   for (int i = 0; i < count; i++) {
     if (int st = gemm_check(A[i], B, m, n, k, r, denoise ? corrA[i] : nullptr, denoise ? corrB[i] : nullptr,
                             denoise ? maxabs[i] : nullptr, lmax, hash ? key[i] : nullptr, target,

@@ -614,30 +614,41 @@ static float plain_form_us(const PlainForm& f, int m, int n, int k, int cus) {
 }
 
 // Whether uwc_gemm_plain_any takes the product: whole k steps, 16-byte output rows (and residual
-// rows), four column scales per load, 32-bit operand offsets within a tile.
-bool uwc_plain_any_fits(int n, int k, int ldc, const void* out, int out_mode, const float* b_scale, const float* res,
-                        const float* out2) {
+// rows), four column scales per load, 32-bit operand offsets within a tile; without an output, whole
+// 128 x 128 tiles.
+bool uwc_plain_any_fits(int m, int n, int k, int ldc, const void* out, int out_mode, const float* b_scale,
+                        const float* res, const float* out2) {
+  if (k % P_BK || k < P_BK || k > (1 << 23)) return false;
+  if (out_mode == P_OUT_NONE) return m % 128 == 0 && n % 128 == 0;
   const bool vec_out = (uintptr_t)out % 16 == 0 && ldc % 4 == 0 && n % 4 == 0 && (uintptr_t)res % 16 == 0 &&
                        (uintptr_t)out2 % 16 == 0;
   const bool vec_scale = (out_mode == P_OUT_I32 && !out2) || (uintptr_t)b_scale % 16 == 0;
-  return out_mode != P_OUT_NONE && vec_out && vec_scale && k % P_BK == 0 && k >= P_BK && k <= (1 << 23);
+  return vec_out && vec_scale;
 }
 
-// A plain GEMM of any m on the form predicted fastest; res (with P_OUT_F32): the residual, out2 (with
-// P_OUT_I32): the dequantized rows beside the sums, both of the output's row stride. Called after the argument checks of uwc_noisy_gemm and uwc_plain_any_fits.
-int uwc_gemm_plain_any(const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
-                       const float* b_scale, const float* res, void* out, float* out2, int out_mode, int ldc,
-                       hipStream_t stream) {
-  const PlainParams p{A, B, m, n, k, a_scale, b_scale, out, ldc, res, out2};
-  const int cus = uwc_cu_count();
+// The form a product takes: the one predicted fastest, or without an output (timing probes) the 4-step
+// ring while a CU has at most one tile and the 2-step one beyond.
+int uwc_plain_form(int m, int n, int k, int out_mode, int out_bytes, int cus) {
+  if (out_mode == P_OUT_NONE) return (long)(m / 128) * (n / 128) <= cus ? 0 : 1;
   int best = 0;
   float best_us = 0.0f;
   for (int i = 0; i < (int)(sizeof(kPlainForms) / sizeof(kPlainForms[0])); i++) {
     const float us = plain_form_us(kPlainForms[i], m, n, k, cus);
     if (i == 0 || us < best_us) best = i, best_us = us;
   }
+  return best;
+}
+
+// A plain GEMM of any m; res (with P_OUT_F32): the residual, out2 (with P_OUT_I32): the dequantized rows
+// beside the sums, both of the output's row stride. Called after the argument checks of uwc_noisy_gemm
+// and uwc_plain_any_fits.
+int uwc_gemm_plain_any(const int8_t* A, const int8_t* B, int m, int n, int k, const float* a_scale,
+                       const float* b_scale, const float* res, void* out, float* out2, int out_mode, int ldc,
+                       hipStream_t stream) {
+  const PlainParams p{A, B, m, n, k, a_scale, b_scale, out, ldc, res, out2};
   const int mode = res ? P_OUT_F32R : out2 ? P_OUT_BOTH : out_mode;
-  switch (best) {
+  const int out_bytes = res || out2 ? 8 : mode == P_OUT_BF16 ? 2 : 4;
+  switch (uwc_plain_form(m, n, k, out_mode, out_bytes, uwc_cu_count())) {
     case 0: plain_any<128, 128, 4>(mode, stream, p); break;
     case 1: plain_any<128, 128, 2>(mode, stream, p); break;
     case 2: plain_any<64, 128, 3>(mode, stream, p); break;

@@ -379,16 +379,23 @@ static void sk_mt(int mt, int out_mode, dim3 grid, dim3 block, size_t lds, hipSt
 #define S2_RG 1
 #endif
 
+// LDS of the X-stationary form: X (padded rows), the reduction buffer and the token scales
+static size_t s2_lds_bytes(int m, int k) {
+  return (((size_t)m * (k + 16) + 15) & ~(size_t)15) + (size_t)8 * S2_RG * 1024 + (size_t)m * 4;
+}
+
+// Whether X fits (else the streaming form runs)
+bool uwc_skinny_resident(int m, int k) { return s2_lds_bytes(m, k) <= S2_MAX_LDS; }
+
 // Called by uwc_noisy_gemm for plain GEMMs (no flags) that uwc_plain_any_fits refuses, with
 // 1 <= m <= 64, k % 64 == 0, out_mode I32 / BF16 / F32, operands already checked (16-byte aligned).
 int uwc_skinny_gemm(const int8_t* X, const int8_t* W, int m, int n, int k, const float* sx, const float* sw,
                     void* out, int out_mode, hipStream_t stream) {
   const int mt = (m + 15) / 16;
-  // X-stationary form when X (padded rows) and the reduction buffer fit in LDS
-  const int xpitch = k + 16;
-  const int RG2 = S2_RG;
-  const size_t lds2 = (((size_t)m * xpitch + 15) & ~(size_t)15) + (size_t)8 * RG2 * 1024 + (size_t)m * 4;
-  if (lds2 <= S2_MAX_LDS) {
+  if (uwc_skinny_resident(m, k)) {
+    const int xpitch = k + 16;
+    const int RG2 = S2_RG;
+    const size_t lds2 = s2_lds_bytes(m, k);
     const int cus = uwc_cu_count();
     const int per_cu = lds2 <= 80 * 1024 ? 2 : 1;
     const long maxg = (long)cus * per_cu;

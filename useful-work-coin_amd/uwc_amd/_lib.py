@@ -29,6 +29,7 @@ SIGNATURES = {
     "uwc_header_sha": [],
     "uwc_noisy_gemm": [vp, vp, i32, i32, i32, i32, vp, vp, vp, i32, vp, vp, vp, i32, vp, vp, vp, i32, i32, vp, vp],
     "uwc_noisy_gemm_many": [i32, vp, vp, i32, i32, i32, i32, vp, vp, vp, i32, vp, vp, vp, i32, vp, vp, vp, i32, i32, vp, vp],
+    "uwc_plain_gemm_route": [i32, i32, i32, i32, i32, i32],
     "uwc_igemm_i32": [vp, vp, i32, i32, i32, vp, vp],
     "uwc_igemm_dequant_f32": [vp, vp, i32, i32, i32, vp, vp, vp, vp],
     "uwc_igemm_dequant_residual_f32": [vp, vp, i32, i32, i32, vp, vp, vp, vp, vp],
