@@ -50,3 +50,12 @@ def test_small_and_odd_products():
     assert route(40, 132, 192) == SKINNY and route(64, 300, 4160) == STREAM
     assert route(40, 4098, 14336) == STREAM and route(64, 300, 4160, NONE) == STAGED
     assert route(0, 4, 128) == -1 and route(4, 4, 100) == -1 and route(4, 4, 128, F32, 2) == -1
+
+
+@pytest.mark.parametrize("m,n,k,out,second,want", [
+    (17, 28672, 4096, F32, 0, 6), (20, 32000, 4096, F32, 0, 6), (384, 12288, 2048, F32, 0, 1), (1280, 4096, 2048, I32, 0, 1),
+    (1536, 3072, 1024, F32, 0, 1), (4096, 1152, 1152, F32, 0, 1), (300, 151936, 2048, I32, 2, 1), (40, 28672, 4096, F32, 0, 4)])
+def test_form_of_products_timed_apart(m, n, k, out, second, want):
+    """Products whose forms differ by 20% and more: the fastest one (wide weights at few rows, a little
+    more than one 128 x 128 tile per CU, a vocabulary's both outputs)."""
+    assert route(m, n, k, out, second) == want

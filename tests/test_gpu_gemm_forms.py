@@ -77,3 +77,72 @@ def test_shapes_left_to_the_other_kernels(dev, m, n, k):
     buf = torch.empty(m * n + 1, dtype=torch.int32, device=dev)
     for out in (buf[:-1].view(m, n), buf[1:].view(m, n)):
         assert np.array_equal(_gemm(A, B, ops.OUT_I32, out).cpu().numpy(), want)
+
+
+# tiles of the forms by number (uwc_plain_gemm_route); forms 0 .. 2 have a kernel for whole tiles and one
+# for ragged ones, 3 .. 8 one for a single row of tiles (weights read once, not kept in the caches) and one
+# for more
+TILES = [(128, 128), (128, 128), (64, 128), (64, 64), (64, 64), (64, 32), (32, 32), (16, 32), (16, 16)]
+EPILOGUES = {"i32": (1, 0), "bf16": (2, 0), "f32": (3, 0), "residual": (3, 1), "both": (1, 2)}
+
+
+def _shape_for(form, first, out, second):
+    """The smallest of a grid of shapes that the rule puts on this form and kernel, on this device."""
+    from uwc_amd import _lib
+    route, (bm, bn) = _lib.lib().uwc_plain_gemm_route, TILES[form]
+    best = None
+    for m in (1, 16, 17, 31, 32, 33, 48, 63, 64, 65, 96, 127, 128, 129, 200, 256, 300, 384, 512, 640, 777, 1024, 1100, 1536, 2048):
+        if ((m <= bm) != first) if form > 2 else (first and m % bm):
+            continue
+        for n in (4, 36, 132, 1028, 2048, 2052, 3072, 4096, 4100, 6144, 8196, 12288, 16384, 20480, 28672):
+            if form <= 2 and (m % bm == 0 and n % bn == 0) != first:
+                continue
+            for k in (128, 256, 384, 640, 1152, 2048, 4096, 6144):
+                if (best is None or m * n * k < best[0]) and route(m, n, k, out, second, 0) == form:
+                    best = (m * n * k, m, n, k)
+    return best and best[1:]
+
+
+@pytest.mark.parametrize("epilogue", list(EPILOGUES))
+@pytest.mark.parametrize("first", [True, False])
+@pytest.mark.parametrize("form", range(9))
+def test_every_form_and_epilogue(dev, form, first, epilogue):
+    """Each instantiation the rule can take, whatever its constants: against the staged kernel's int32
+    sums and the oracle's roundings."""
+    from uwc_amd import _lib, ops
+    out, second = EPILOGUES[epilogue]
+    shape = _shape_for(form, first, out, second)
+    assert shape or epilogue != "f32", "a form that the rule never takes"
+    if shape is None:
+        pytest.skip("the rule does not take this kernel with this epilogue")
+    m, n, k = shape
+    A, B = _rand(dev, m + k, m, k), _rand(dev, n + 3 * k, n, k)
+    ref = _gemm(A, B, ops.OUT_I32, torch.empty((m, n), dtype=torch.int32, device=dev), flags=ops.FLAG_TILE128)
+    rng = np.random.default_rng(form)
+    sx = (rng.random(m, dtype=np.float32) * 1e-2 + 1e-4).astype(np.float32)
+    sw = (rng.random(n, dtype=np.float32) * 1e-3 + 1e-5).astype(np.float32)
+    sxt, swt = torch.from_numpy(sx).to(dev), torch.from_numpy(sw).to(dev)
+    acc = ref.cpu().numpy()
+    st = torch.cuda.current_stream().cuda_stream
+    if epilogue == "residual":
+        x = rng.standard_normal((m, n)).astype(np.float32)
+        Y = torch.empty((m, n), device=dev)
+        xt = torch.from_numpy(x).to(dev)
+        _lib.call("uwc_igemm_dequant_residual_f32", A.data_ptr(), B.data_ptr(), m, n, k, sxt.data_ptr(), swt.data_ptr(),
+                  xt.data_ptr(), Y.data_ptr(), st)
+        assert np.array_equal(Y.cpu().numpy().view(np.uint32), (x + O.dequant(acc, sx, sw)).view(np.uint32))
+    elif epilogue == "both":
+        C, Y = torch.empty((m, n), dtype=torch.int32, device=dev), torch.empty((m, n), device=dev)
+        _lib.call("uwc_igemm_i32_dequant_f32", A.data_ptr(), B.data_ptr(), m, n, k, sxt.data_ptr(), swt.data_ptr(),
+                  C.data_ptr(), Y.data_ptr(), st)
+        assert torch.equal(C, ref)
+        assert np.array_equal(Y.cpu().numpy().view(np.uint32), O.dequant(acc, sx, sw).view(np.uint32))
+    else:
+        dt = {"i32": torch.int32, "bf16": torch.bfloat16, "f32": torch.float32}[epilogue]
+        Y = _gemm(A, B, out, torch.empty((m, n), dtype=dt, device=dev), sx=sxt, sw=swt)
+        if epilogue == "i32":
+            assert torch.equal(Y, ref)
+        elif epilogue == "f32":
+            assert np.array_equal(Y.cpu().numpy().view(np.uint32), O.dequant(acc, sx, sw).view(np.uint32))
+        else:
+            assert np.array_equal(Y.cpu().view(torch.int16).numpy().view(np.uint16), O.scale_bf16(acc, sx, sw))

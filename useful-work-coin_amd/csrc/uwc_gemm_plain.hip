@@ -583,34 +583,43 @@ int uwc_gemm_plain(int cfg, const int8_t* A, const int8_t* B, int m, int n, int 
 }
 
 // The forms the automatic choice takes, with their tile, the workgroups a CU holds at once (by LDS)
-// and the constants of their time in us: start + (k / 128) max(lat rounds, load x) + per_tile (x - 1)
+// and the constants of their time in us:
+//   start + max((k / 128) max(lat rounds, load x) + per_tile (x - 1), stream MB(B)) + store MB(out)
 // for x tiles per CU in `rounds` rounds of `occ`. lat is what a k step of one tile takes (its wave's
-// or its barrier's chain), load what it costs a CU that has other tiles to work on, per_tile a
-// tile's share of the epilogues. Fitted to 242 shapes (m 1 .. 3000, n 1152 .. 20480, k 1152 .. 14336,
-// every form timed at each): the form with the least predicted time is on average within 1% of the
-// fastest one and within 3.4% at nine shapes of ten (16% at worst); dropping any of the nine forms
-// costs up to 29% somewhere.
+// or its barrier's chain), load what it costs a CU that has other tiles to work on, per_tile what else a
+// tile after the first costs, stream what reading the n x k weight from HBM takes with the bytes this form
+// keeps in flight, store what writing the output (and reading a residual) adds. Fitted to 4660 products
+// (m 1 .. 8192; the linears and heads of two models, 33 other n x k and 1278 random ones, n 4 .. 151936, k
+// 128 .. 14336; fp32 out, with a residual, with both outputs; weights rotated over 1.3 GB, every form timed
+// at each): the form with the least predicted time is on average within 0.8% of the fastest one, within
+// 2.3% at nine products of ten, 13% at 99 of 100 and 67% at worst (666 x 10828 x 384 with both outputs);
+// fitted to three quarters of the n x k, within 0.7 to 1.3% on average on the fourth. Without the stream
+// and store terms it was 1.7%, 5.7%, 25% and 64%, and slower than the kernels before it at 17 x 28672 x
+// 4096 (23.1 us; 29.1, now 22.7), 384 x 12288 x 2048 (21.9; 26.9, now 21.9) and 4096 x 1152 x 1152 (11.0;
+// 14.3, now 11.1); 300 x 151936 x 2048 with both outputs 224 -> 194.
 struct PlainForm {
   int bm, bn, occ;
-  float start, lat, load, per_tile;
+  float start, lat, load, per_tile, stream, store;
 };
 static const PlainForm kPlainForms[] = {
-    {128, 128, 1, 4.98f, 0.4185f, 0.0f, 7.03f},      // plain, 4-step ring
-    {128, 128, 2, 2.58f, 0.7405f, 0.0f, 6.27f},      // plain, 2-step ring
-    {64, 128, 2, 3.17f, 0.3420f, 0.3168f, 1.26f},    // plain, 3-step ring
-    {64, 64, 4, 3.17f, 0.2932f, 0.1903f, 0.50f},     // 2 waves
-    {64, 64, 2, 3.43f, 0.0f, 0.1882f, 1.05f},        // 4 waves
-    {64, 32, 1, 3.25f, 0.1306f, 0.0f, 1.65f},        // 4 waves, 2 stages
-    {32, 32, 2, 2.85f, 0.0940f, 0.0842f, 0.36f},     // 4 waves, 2 stages
-    {16, 32, 3, 2.91f, 0.0750f, 0.0622f, 0.12f},     // 4 waves, 2 stages
-    {16, 16, 3, 2.84f, 0.0541f, 0.0388f, 0.20f},     // 4 waves, 3 stages
+    {128, 128, 1, 2.926f, 0.4991f, 0.5102f, 0.6004f, 0.2037f, 0.2054f},  // plain, 4-step ring
+    {128, 128, 2, 2.024f, 0.871f, 0.1203f, 0.3671f, 0.1948f, 0.197f},    // plain, 2-step ring
+    {64, 128, 2, 2.651f, 0.4285f, 0.3284f, 0.0f, 0.2202f, 0.1739f},      // plain, 3-step ring
+    {64, 64, 4, 3.114f, 0.4166f, 0.2283f, 0.2235f, 0.1818f, 0.1077f},    // 2 waves
+    {64, 64, 2, 3.068f, 0.1199f, 0.238f, 0.00318f, 0.1701f, 0.1348f},    // 4 waves
+    {64, 32, 1, 2.671f, 0.0681f, 0.1599f, 1.263f, 0.1958f, 0.3708f},     // 4 waves, 2 stages
+    {32, 32, 2, 2.285f, 0.1266f, 0.1197f, 0.01813f, 0.1719f, 0.3065f},   // 4 waves, 2 stages
+    {16, 32, 3, 2.193f, 0.03946f, 0.1232f, 0.0f, 0.1494f, 0.3613f},      // 4 waves, 2 stages
+    {16, 16, 3, 2.258f, 0.04214f, 0.07793f, 0.0f, 0.1227f, 0.3837f},     // 4 waves, 3 stages
 };
 
-static float plain_form_us(const PlainForm& f, int m, int n, int k, int cus) {
+// out_bytes: what an element of the output moves (its own bytes, a residual's, a second output's)
+static float plain_form_us(const PlainForm& f, int m, int n, int k, int out_bytes, int cus) {
   const long tiles = (long)((m + f.bm - 1) / f.bm) * ((n + f.bn - 1) / f.bn);
   const long x = (tiles + cus - 1) / cus, rounds = (x + f.occ - 1) / f.occ;
   const float step = f.lat * rounds > f.load * x ? f.lat * rounds : f.load * x;
-  return f.start + (k / P_BK) * step + f.per_tile * (x - 1);
+  const float work = (k / P_BK) * step + f.per_tile * (x - 1), stream = f.stream * 1e-6f * n * k;
+  return f.start + (work > stream ? work : stream) + f.store * 1e-6f * m * n * out_bytes;
 }
 
 // Whether uwc_gemm_plain_any takes the product: whole k steps, 16-byte output rows (and residual
@@ -633,7 +642,7 @@ int uwc_plain_form(int m, int n, int k, int out_mode, int out_bytes, int cus) {
   int best = 0;
   float best_us = 0.0f;
   for (int i = 0; i < (int)(sizeof(kPlainForms) / sizeof(kPlainForms[0])); i++) {
-    const float us = plain_form_us(kPlainForms[i], m, n, k, cus);
+    const float us = plain_form_us(kPlainForms[i], m, n, k, out_bytes, cus);
     if (i == 0 || us < best_us) best = i, best_us = us;
   }
   return best;
