@@ -59,3 +59,16 @@ def test_form_of_products_timed_apart(m, n, k, out, second, want):
     """Products whose forms differ by 20% and more: the fastest one (wide weights at few rows, a little
     more than one 128 x 128 tile per CU, a vocabulary's both outputs)."""
     assert route(m, n, k, out, second) == want
+
+
+@pytest.mark.parametrize("m,n,k", [(1 << 28, 4, 128), ((1 << 28) + 5, 16, 1152), ((1 << 30) + 1, 4, 128), (1, 1 << 24, 4096),
+                                   (4, 1 << 28, 128), (1 << 20, 1 << 16, 128), (1 << 24, 28672, 2048)])
+@pytest.mark.parametrize("second", [0, 1])
+def test_form_grids_hold_fewer_than_2_to_32_threads(m, n, k, second):
+    """Very long or wide products take tiles whose grid one launch can hold."""
+    tiles = [(128, 128), (128, 128), (64, 128), (64, 64), (64, 64), (64, 32), (32, 32), (16, 32), (16, 16)]
+    f = route(m, n, k, F32, second)
+    if f in (LARGE, COLUMNS):
+        return
+    bm, bn = tiles[f]
+    assert -(-m // bm) * -(-n // bn) * 256 < 1 << 32

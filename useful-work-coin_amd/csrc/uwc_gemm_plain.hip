@@ -615,7 +615,7 @@ static const PlainForm kPlainForms[] = {
 
 // out_bytes: what an element of the output moves (its own bytes, a residual's, a second output's)
 static float plain_form_us(const PlainForm& f, int m, int n, int k, int out_bytes, int cus) {
-  const long tiles = (long)((m + f.bm - 1) / f.bm) * ((n + f.bn - 1) / f.bn);
+  const long tiles = ((m + (long)f.bm - 1) / f.bm) * ((n + (long)f.bn - 1) / f.bn);
   const long x = (tiles + cus - 1) / cus, rounds = (x + f.occ - 1) / f.occ;
   const float step = f.lat * rounds > f.load * x ? f.lat * rounds : f.load * x;
   const float work = (k / P_BK) * step + f.per_tile * (x - 1), stream = f.stream * 1e-6f * n * k;
@@ -642,7 +642,11 @@ int uwc_plain_form(int m, int n, int k, int out_mode, int out_bytes, int cus) {
   int best = 0;
   float best_us = 0.0f;
   for (int i = 0; i < (int)(sizeof(kPlainForms) / sizeof(kPlainForms[0])); i++) {
-    const float us = plain_form_us(kPlainForms[i], m, n, k, out_bytes, cus);
+    const PlainForm& f = kPlainForms[i];
+    // a grid of 2^32 threads or more would be cut off without an error (2^28 rows of 4 columns on small tiles)
+    const u64 tiles = (u64)((m + (long)f.bm - 1) / f.bm) * (u64)((n + (long)f.bn - 1) / f.bn);
+    if (i > 0 && tiles * P_THREADS > 0xFFFFFFFFull) continue;
+    const float us = plain_form_us(f, m, n, k, out_bytes, cus);
     if (i == 0 || us < best_us) best = i, best_us = us;
   }
   return best;
