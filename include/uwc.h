@@ -127,7 +127,7 @@ int uwc_igemm_dequant_residual_f32(const int8_t* A, const int8_t* B, int m, int 
 
 /* Both C = A * B^T (int32) and Y = fmul(fmul(f32(C), sx[i]), sw[j]) (fp32), m x n each: one epilogue
  * writes both where the 256 x 256 tiles do not take the shape, else uwc_igemm_i32 and
- * uwc_dequant_f32; the same bits either way.
+ * uwc_dequant_f32; the same bits either way. Y must not overlap C.
  * Replaces DetLinear.int_gemm + dequant of the lm_head: runtime/detrt/qwen3.py:106-126, 300-311. */
 int uwc_igemm_i32_dequant_f32(const int8_t* A, const int8_t* B, int m, int n, int k, const float* sx, const float* sw,
                               int32_t* C, float* Y, hipStream_t stream);

@@ -205,3 +205,13 @@ def test_loader_refuses_library_of_another_header(tmp_path, monkeypatch):
     monkeypatch.setattr(_lib, "_LIB", None)
     with pytest.raises(ImportError, match="another include/uwc.h"):
         _lib.lib()
+
+
+@pytest.mark.parametrize("off", [0, 16, 256 * 256 * 4 - 16, -16])
+def test_sums_and_dequantized_rows_may_not_overlap(off):
+    """uwc_igemm_i32_dequant_f32 writes C and Y: overlapping ones are refused before any launch."""
+    from uwc_amd import _lib
+    L = _lib.lib()
+    fake, other = ctypes.c_void_p(1 << 20), ctypes.c_void_p((1 << 20) + off)
+    assert L.uwc_igemm_i32_dequant_f32(fake, fake, 256, 256, 128, fake, fake, fake, other, None) == -1
+    assert "overlaps" in L.uwc_last_error().decode()

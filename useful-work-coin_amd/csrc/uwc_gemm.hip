@@ -514,6 +514,8 @@ extern "C" int uwc_igemm_i32_dequant_f32(const int8_t* A, const int8_t* B, int m
   if (int st = gemm_check(A, B, m, n, k, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, 0, sx, sw, Y,
                           OUT_F32, 0))
     return st;
+  const uintptr_t ca = (uintptr_t)C, ya = (uintptr_t)Y, bytes = (uintptr_t)m * (uintptr_t)n * 4;
+  if (ca < ya + bytes && ya < ca + bytes) return uwc_fail("%s: Y overlaps C", fn);
   if (large_tiles(m, n, k, aligned16(C) && n % 4 == 0, uwc_cu_count()) == LARGE_NONE &&
       uwc_plain_any_fits(m, n, k, n, C, OUT_I32, sw, nullptr, Y))
     return uwc_gemm_plain_any(A, B, m, n, k, sx, sw, nullptr, C, Y, OUT_I32, n, stream);

@@ -643,7 +643,7 @@ int uwc_plain_form(int m, int n, int k, int out_mode, int out_bytes, int cus) {
   float best_us = 0.0f;
   for (int i = 0; i < (int)(sizeof(kPlainForms) / sizeof(kPlainForms[0])); i++) {
     const PlainForm& f = kPlainForms[i];
-    // a grid of 2^32 threads or more would be cut off without an error (2^28 rows of 4 columns on small tiles)
+    // a grid of 2^32 threads or more would be cut off without an error (2^28 rows of 16 columns on 16 x 16 tiles)
     const u64 tiles = (u64)((m + (long)f.bm - 1) / f.bm) * (u64)((n + (long)f.bn - 1) / f.bn);
     if (i > 0 && tiles * P_THREADS > 0xFFFFFFFFull) continue;
     const float us = plain_form_us(f, m, n, k, out_bytes, cus);
