@@ -517,6 +517,34 @@ def test_quantizing_row_kernels_widths(dev, rows, k, bs):
     assert np.array_equal(q.cpu().numpy()[pick], rq) and np.array_equal(_u32(s)[pick], _u32(rs))
 
 
+def test_one_call_paths_take_weights_only_as_they_lie(dev):
+    """layer_fused and final_logits over reassigned weights: strided scales give the same rows, a strided
+    or float weight is refused as by the op-by-op path, and so are Hadamard blocks that do not divide."""
+    from uwc_amd import detgpu
+    cfg = dict(D=256, H=4, Hkv=2, hd=64, I=384, L=1, V=512, eps=1e-6, Bs=64, max_pos=70, theta=1e4, arch=1)
+    m = detgpu.DetModel.random(cfg, seed=5, device=dev)
+    L = m.layers[0]
+    x = torch.randn((140, 256), device=dev)
+    runs = [(lin, lambda: detgpu.layer_fused(m, L, x, 2, 70)) for lin in (L["qkv"], L["gu"])]
+    runs.append((m.lm_head, lambda: torch.cat(detgpu.final_logits(m, x), 1)))
+    for lin, run in runs:
+        want, Wq, sw, bs = run(), lin.Wq, lin.sw, lin.bs
+        wide = torch.zeros((lin.n, 2), device=dev)
+        wide[:, 0] = sw
+        lin.sw = wide[:, 0]
+        assert torch.equal(run(), want)
+        lin.sw = sw
+        for bad in (Wq.t().contiguous().t(), Wq.float()):
+            lin.Wq = bad
+            with pytest.raises(AssertionError):
+                run()
+        lin.Wq, lin.bs = Wq, 512
+        with pytest.raises(AssertionError):
+            run()
+        lin.bs = bs
+        assert torch.equal(run(), want)
+
+
 @pytest.mark.parametrize("rows,words", [(63, 256), (65, 256), (64, 300), (130, 1024), (4097, 300), (16385, 300)])
 def test_sha_row_roots_workgroup_edges(dev, rows, words):
     """Row trees just under, at and past the 64 rows of a workgroup, at one, two and four blocks per row."""

@@ -435,16 +435,25 @@ class DetModel:
 _INT_GEMM = DetLinear.int_gemm  # a layer whose linears carry another one (a miner's) runs op by op
 
 
+def _plain(lin, dev) -> bool:
+    """Whether a library call may take the linear's weights as they lie in memory: a DetLinear that does
+    not mine, with its own int_gemm, whose weights and scales (which may have been reassigned) have its
+    shape, type and device and are contiguous, and whose Hadamard blocks divide its rows. The op-by-op path
+    copies or refuses what is not."""
+    return (type(lin) is DetLinear and not (lin.mine and lin.mw is not None) and
+            getattr(lin.int_gemm, "__func__", None) is _INT_GEMM and
+            lin.Wq.dtype == torch.int8 and lin.Wq.shape == (lin.n, lin.k) and lin.Wq.is_contiguous() and
+            lin.Wq.device == dev and lin.sw.dtype == F32 and lin.sw.shape == (lin.n,) and lin.sw.is_contiguous() and
+            lin.sw.device == dev and not (lin.bs > 1 and lin.k % lin.bs))
+
+
 def _layer_call(m, L, x, B, T, out):
-    """layer_fused as one library call, or None for what that call does not take: linears that mine
-    or whose int_gemm was replaced, operands that are not contiguous float32 of the model's shapes
-    on x's device."""
+    """layer_fused as one library call, or None for what that call does not take: linears that are
+    not _plain, operands that are not contiguous float32 of the model's shapes on x's device."""
     H, Hkv, dev = m.H, m.Hkv, x.device
     qkv, o, gu, down = L["qkv"], L["o"], L["gu"], L["down"]
-    for lin in (qkv, o, gu, down):
-        if type(lin) is not DetLinear or (lin.mine and lin.mw is not None) or \
-                getattr(lin.int_gemm, "__func__", None) is not _INT_GEMM or lin.Wq.device != dev:
-            return None
+    if not all(_plain(lin, dev) for lin in (qkv, o, gu, down)):
+        return None
     if x.dim() != 2 or qkv.n % (H + 2 * Hkv):
         return None
     N, D = x.shape
@@ -558,8 +567,7 @@ def final_logits(m, x: torch.Tensor):
     logits), the rows DetQwen3.logprobs starts from (qwen3.py:300-311)."""
     lin = m.lm_head
     q, s = rmsnorm_quant(x.reshape(-1, m.D), m.norm, m.eps, lin.bs)
-    if type(lin) is not DetLinear or (lin.mine and lin.mw is not None) or \
-            getattr(lin.int_gemm, "__func__", None) is not _INT_GEMM:
+    if not _plain(lin, q.device):
         acc = lin.int_gemm(q)
         return acc, dequant(acc, s, lin.sw)
     acc = torch.empty((q.shape[0], lin.n), dtype=torch.int32, device=q.device)
