@@ -215,3 +215,17 @@ def test_sums_and_dequantized_rows_may_not_overlap(off):
     fake, other = ctypes.c_void_p(1 << 20), ctypes.c_void_p((1 << 20) + off)
     assert L.uwc_igemm_i32_dequant_f32(fake, fake, 256, 256, 128, fake, fake, fake, other, None) == -1
     assert "overlaps" in L.uwc_last_error().decode()
+
+
+@pytest.mark.parametrize("kwargs,msg", [(dict(k=30), "multiple of 64"), (dict(W=None), "null"), (dict(rows=0), "empty"),
+                                        (dict(q=4), "16-byte aligned"), (dict(Y=None), "null")])
+def test_det_linear_refuses_before_it_quantizes(kwargs, msg):
+    """uwc_det_linear_f32 refuses what its GEMM would before the quantizer is launched."""
+    from uwc_amd import _lib
+    L = _lib.lib()
+    a = dict(rows=4, k=64, W=0, q=0, Y=0)
+    a.update(kwargs)
+    at = lambda v: None if v is None else ctypes.c_void_p((1 << 20) + v)
+    st = L.uwc_det_linear_f32(at(0), a["rows"], a["k"], 0, at(a["W"]), 8, at(0), at(a["q"]), at(0), at(a["Y"]), None)
+    assert st == -1
+    assert "uwc_det_linear_f32" in L.uwc_last_error().decode() and msg in L.uwc_last_error().decode()

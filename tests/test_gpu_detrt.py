@@ -175,3 +175,14 @@ def test_dequant_every_layout(dev, m, n):
     sw = rng.uniform(1e-6, 1e-2, n).astype(np.float32)
     y = detrt.dequant(torch.from_numpy(acc).to(dev), torch.from_numpy(sx).to(dev), torch.from_numpy(sw).to(dev))
     assert np.array_equal(y.cpu().numpy().view(np.uint32), O.dequant(acc, sx, sw).view(np.uint32))
+
+
+def test_det_linear_refuses_undividing_blocks(dev):
+    """Hadamard blocks that do not divide k raise quant_act's AssertionError, a k the GEMM does not take RuntimeError."""
+    from uwc_amd import detrt
+    lay = detrt.DetLinear.from_quantized(torch.zeros((8, 192), dtype=torch.int8, device=dev), torch.ones(8, device=dev), 128)
+    with pytest.raises(AssertionError):
+        lay(torch.zeros((3, 192), device=dev))
+    with pytest.raises(RuntimeError):
+        detrt.DetLinear.from_quantized(torch.zeros((8, 96), dtype=torch.int8, device=dev), torch.ones(8, device=dev), 32)(
+            torch.zeros((3, 96), device=dev))

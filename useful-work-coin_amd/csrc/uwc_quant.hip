@@ -343,6 +343,11 @@ extern "C" int uwc_dequant_f32(const int32_t* acc, const float* sx, const float*
 
 extern "C" int uwc_det_linear_f32(const float* x, int rows, int k, int bs, const int8_t* W, int n, const float* sw,
                                   int8_t* q, float* scale, float* Y, hipStream_t stream) {
+  const char* fn = "uwc_det_linear_f32";
+  // what the GEMM would refuse after the rows were quantized (scale may lie behind q, off a multiple of 4)
+  if (k % 64) return uwc_fail("%s: k=%d must be a multiple of 64", fn, k);
+  if (!W || !sw || !Y || rows <= 0 || n <= 0) return uwc_fail("%s: null or empty arguments", fn);
+  if (((uintptr_t)q | (uintptr_t)W) & 15) return uwc_fail("%s: q and W must be 16-byte aligned", fn);
   if (int st = uwc_quant_act_f32(x, rows, k, bs, 64, q, scale, stream)) return st;
   return uwc_igemm_dequant_f32(q, W, rows, n, k, scale, sw, Y, stream);
 }

@@ -129,6 +129,8 @@ class DetLinear:
             rows = rows.contiguous()
             if rows.dtype != torch.float32:
                 rows = rows.to(torch.float32)
+            if self.bs > 1 and k % self.bs:
+                raise AssertionError(f"quant_act: bs={self.bs} must divide k={k}")
             m, dev = rows.shape[0], rows.device
             y = torch.empty((m, n), dtype=torch.float32, device=dev)
             # the quantized rows, then their scales (k % 64 == 0: both aligned)
