@@ -523,8 +523,6 @@ void plain_out(int out_mode, hipStream_t s, const PlainParams& p) {
     case P_OUT_NONE: plain_go<BM, BN, S, SPREAD, false, P_OUT_NONE>(s, p); break;
     case P_OUT_I32: plain_go<BM, BN, S, SPREAD, false, P_OUT_I32>(s, p); break;
     case P_OUT_BF16: plain_go<BM, BN, S, SPREAD, false, P_OUT_BF16>(s, p); break;
-    case P_OUT_F32R: plain_go<BM, BN, S, SPREAD, false, P_OUT_F32R>(s, p); break;
-    case P_OUT_BOTH: plain_go<BM, BN, S, SPREAD, false, P_OUT_BOTH>(s, p); break;
     default: plain_go<BM, BN, S, SPREAD, false, P_OUT_F32>(s, p); break;
   }
 }
@@ -532,7 +530,11 @@ void plain_out(int out_mode, hipStream_t s, const PlainParams& p) {
 // any m, n % 4 == 0 (with an output)
 template <int BM, int BN, int S>
 void plain_any(int out_mode, hipStream_t s, const PlainParams& p) {
-  if (p.m % BM == 0 && p.n % BN == 0) return plain_out<BM, BN, S, true>(out_mode, s, p);
+  if (p.m % BM == 0 && p.n % BN == 0) {
+    if (out_mode == P_OUT_F32R) return plain_go<BM, BN, S, true, false, P_OUT_F32R>(s, p);
+    if (out_mode == P_OUT_BOTH) return plain_go<BM, BN, S, true, false, P_OUT_BOTH>(s, p);
+    return plain_out<BM, BN, S, true>(out_mode, s, p);
+  }
   switch (out_mode) {
     case P_OUT_I32: plain_go<BM, BN, S, true, true, P_OUT_I32>(s, p); break;
     case P_OUT_BF16: plain_go<BM, BN, S, true, true, P_OUT_BF16>(s, p); break;

@@ -160,18 +160,11 @@ __global__ void __launch_bounds__(512) skinny_gemm_kernel(const i8* __restrict__
 //     one batch ahead across row-block boundaries with statically known wait counts;
 //   * at the end of a row block the KS partials of each row group are summed through LDS, one
 //     token group at a time (integer sums: the split cannot change the result).
-typedef const void __attribute__((address_space(1)))* s2_gptr;
 typedef void __attribute__((address_space(3)))* s2_lptr;
 
 // One wave-wide 16-byte-per-lane DMA into LDS at lds + 16 lane (lds wave-uniform, in M0).
 __device__ __forceinline__ void s2_dma16(const void* g, u32 lds) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
-}
-// The same with the non-temporal hint, for W: every weight byte is read once per call, and
-// cached normally its stream evicts X and the scales, which every workgroup of the XCD rereads
-// (Llama-3.1-8B decode layer at M = 1: 51.0 -> 47.7 us).
-__device__ __forceinline__ void s2_dma16_nt(const void* g, u32 lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "s"(lds) : "memory", "m0");
 }
 
 // Workgroup barrier for LDS traffic only: waits for this wave's LDS operations, not for its
