@@ -1,9 +1,9 @@
-"""GPU parity of the skinny GEMM path (m <= 64: decode and small batches, BASELINE configs 1 and 4)
-through the C-ABI: exact int32 products against the CPU oracle and against the 128 x 128
-tiled kernel (UWC_FLAG_TILE128), every token count 1..64 boundary, ragged n and k, and the
-fp32 / bf16 dequant epilogues bit for bit (runtime/detrt/qwen3.py:106-126). Both skinny forms
-run: the X-stationary one (X staged in LDS, m * (k + 16) bytes up to ~150 KB) and the streaming
-one for larger X (e.g. 40 x 14336, 64 x 4096)."""
+"""GPU parity of plain GEMMs of few rows (m <= 64: decode and small batches)
+through the C-ABI: exact int32 products against the CPU oracle and against the 128 x 128 tiled kernel
+(UWC_FLAG_TILE128), every token count 1..64 boundary, ragged n and k, and the fp32 / bf16 dequant
+epilogues bit for bit (runtime/detrt/qwen3.py:106-126). Most shapes run on the plain kernels' small
+tiles. The skinny kernels take what those do not (k % 128, n % 4, an unaligned output): X in LDS up to
+160 KB, streamed past that; test_skinny_kernels_* name their shapes by the route."""
 import numpy as np
 import pytest
 import torch
@@ -84,3 +84,47 @@ def test_skinny_det_linear_decode(dev):
     y = lay(torch.from_numpy(x).to(dev))
     _, _, _, want = O.det_linear(x, Wq, sw, bs)
     assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+# (m, n, k, route): X in LDS (18) and streamed (19), one and two 16-column groups per workgroup (n from
+# 32753 on), four and eight waves, fewer k steps than the waves take at once
+SKINNY_SHAPES = [(19, 1002, 1024, 18), (5, 6, 128, 18), (64, 301, 1088, 18), (40, 132, 192, 18), (33, 70, 4672, 18),
+                 (64, 300, 4160, 19), (40, 4098, 14336, 19), (17, 9, 9920, 19), (33, 8210, 4928, 19), (24, 32770, 6976, 19)]
+
+
+@pytest.mark.parametrize("m,n,k,route", SKINNY_SHAPES)
+def test_skinny_kernels_every_output(dev, m, n, k, route):
+    """Both skinny kernels with every output, against the oracle (the tiled kernel where that is long)."""
+    from uwc_amd import _lib, ops
+    assert _lib.lib().uwc_plain_gemm_route(m, n, k, ops.OUT_I32, 0, 0) == route
+    g = torch.Generator(device=dev)
+    g.manual_seed(m + n + k)
+    A = torch.randint(-128, 128, (m, k), dtype=torch.int8, device=dev, generator=g)
+    B = torch.randint(-128, 128, (n, k), dtype=torch.int8, device=dev, generator=g)
+    acc = _gemm(A, B, ops.OUT_I32, flags=ops.FLAG_TILE128).cpu().numpy()
+    if m * n * k <= 1 << 27:
+        assert np.array_equal(acc, O.igemm(A.cpu().numpy(), B.cpu().numpy()))
+    assert np.array_equal(_gemm(A, B, ops.OUT_I32).cpu().numpy(), acc)
+    rng = np.random.default_rng(m + n)
+    sx = (rng.random(m, dtype=np.float32) * 1e-2 + 1e-4).astype(np.float32)
+    sw = (rng.random(n, dtype=np.float32) * 1e-3 + 1e-5).astype(np.float32)
+    sxt, swt = torch.from_numpy(sx).to(dev), torch.from_numpy(sw).to(dev)
+    Y = _gemm(A, B, ops.OUT_F32, sx=sxt, sw=swt)
+    assert np.array_equal(Y.cpu().numpy().view(np.uint32), O.dequant(acc, sx, sw).view(np.uint32))
+    Yb = _gemm(A, B, ops.OUT_BF16, sx=sxt, sw=swt)
+    assert np.array_equal(Yb.cpu().view(torch.int16).numpy().view(np.uint16), O.scale_bf16(acc, sx, sw))
+
+
+@pytest.mark.parametrize("m,n,k", [(8, 512, 1024), (64, 4096, 4096)])
+def test_skinny_kernels_unaligned_output(dev, m, n, k):
+    """An output 4 bytes off a 16-byte boundary, X in LDS and streamed: rows as into an aligned one, nothing
+    written around them."""
+    from uwc_amd import _lib, ops
+    g = torch.Generator(device=dev)
+    g.manual_seed(n)
+    A = torch.randint(-128, 128, (m, k), dtype=torch.int8, device=dev, generator=g)
+    B = torch.randint(-128, 128, (n, k), dtype=torch.int8, device=dev, generator=g)
+    buf = torch.full((m * n + 9,), -77, dtype=torch.int32, device=dev)
+    _lib.call("uwc_igemm_i32", A.data_ptr(), B.data_ptr(), m, n, k, buf.data_ptr() + 4, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(buf[1:m * n + 1].view(m, n), _gemm(A, B, ops.OUT_I32))
+    assert int(buf[0]) == -77 and bool((buf[m * n + 1:] == -77).all())

@@ -1,12 +1,9 @@
-"""GPU parity of the DMA-streamed skinny GEMM form (m <= 64, k % 1024 == 0: W through an LDS
-ring by DMA, X of a token group resident in LDS or streamed with W) through the C-ABI. Shapes are
-picked to reach every branch of its plan: one and two token groups, X resident or streamed (8 or
-16 X rows per entry), one and two partials buffers, ring depths 4..6, ragged n (a partial last
-16-row block), n as small as one block, many blocks per workgroup (a weight-scale table of several
-DMAs), 1, 2, 3, 4, 14 and 30 chunks of 1 KB per row, and the odd m that must fall back to the
-other forms. Each result is compared with the 128 x 128 tiled kernel
-(UWC_FLAG_TILE128) and, where it is cheap, with the CPU oracle; the fp32 / bf16 epilogues bit for
-bit with the oracle's dequant (runtime/detrt/qwen3.py:106-126)."""
+"""GPU parity of plain GEMMs of few rows (m <= 64) over k % 1024 == 0 through the C-ABI, most of them on the
+small tiles of the plain kernels whose waves split k and read W past the caches where one row of tiles
+reads it once: one to four tile rows, ragged n, n as small as one tile, a vocabulary's columns, k from
+fewer steps than the waves take at once to 30 KB rows, odd m. Each result is compared with the 128 x 128
+tiled kernel (UWC_FLAG_TILE128) and, where it is cheap, with the CPU oracle; the fp32 / bf16 epilogues bit
+for bit with the oracle's dequant (runtime/detrt/qwen3.py:106-126)."""
 import numpy as np
 import pytest
 import torch
@@ -28,27 +25,25 @@ def _gemm(A, B, out_mode, flags=0, sx=None, sw=None):
     return out
 
 
-# (m, n, k): token groups / partials buffers / ring depth the plan gives on a 256-CU part
 SHAPES = [
-    (1, 4, 1024),        # one block, one workgroup busy
-    (3, 20, 1024),       # partial second block
-    (16, 1000, 2048),    # 63 blocks, the last one partial
-    (19, 1000, 1024),    # two token tiles in one group
-    (34, 300, 4096),     # two token groups of 17, one partials buffer
-    (48, 96, 2048),      # two groups of 24
-    (64, 96, 2048),      # two groups of 32, one partials buffer
-    (64, 1000, 1024),    # two groups, ring depth 5
-    (8, 4096, 14336),    # 14 chunks per row, two groups of 4
-    (8, 64, 3072),       # 3 chunks per row
-    (1, 28672, 4096),    # 7 blocks per workgroup
-    (64, 6144, 2048),
+    (1, 4, 1024),        # one tile
+    (3, 20, 1024),       # a partial last tile
+    (16, 1000, 2048),    # one full tile row
+    (19, 1000, 1024),    # two tile rows of 16, the second of 3
+    (34, 300, 4096),
+    (48, 96, 2048),
+    (64, 96, 2048),
+    (64, 1000, 1024),
+    (8, 4096, 14336),    # 112 k steps
+    (8, 64, 3072),
+    (1, 28672, 4096),    # seven tiles per CU
+    (64, 6144, 2048),    # a 64-row MLP up projection
     (32, 6144, 4096),    # Llama-3.1-8B qkv at M = 32
-    (33, 300, 4096),     # odd m whose X does not fit one group: the other forms
-    # X streamed through the ring with W (too large to stay resident)
-    (32, 4096, 14336),   # Llama-3.1-8B down at M = 32: two groups of 16, 16 X rows per entry
-    (9, 1000, 14336),    # odd m, one group of 9 (rows 9..15 of the entry repeat row 8)
-    (24, 2000, 14336),   # two groups of 12
-    (6, 256, 30720),     # 8 X rows per entry, 30 chunks per row
+    (33, 300, 4096),
+    (32, 4096, 14336),   # Llama-3.1-8B down at M = 32
+    (9, 1000, 14336),
+    (24, 2000, 14336),
+    (6, 256, 30720),     # 240 k steps
 ]
 
 
@@ -67,7 +62,7 @@ def test_skinny_dma_int32(dev, m, n, k):
 
 
 def test_skinny_dma_many_blocks_per_workgroup(dev):
-    """38 blocks per workgroup: the weight-scale table takes three DMAs; int32 and fp32 out."""
+    """A vocabulary's columns at two rows: many tiles per CU; int32 and fp32 out."""
     from uwc_amd import ops
     m, n, k = 2, 151936, 1024
     g = torch.Generator(device=dev)
