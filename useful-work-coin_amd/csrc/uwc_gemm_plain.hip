@@ -615,13 +615,13 @@ static const PlainForm kPlainForms[] = {
     {16, 16, 3, 2.258f, 0.04214f, 0.07793f, 0.0f, 0.1227f, 0.3837f},     // 4 waves, 3 stages
 };
 
-// out_bytes: what an element of the output moves (its own bytes, a residual's, a second output's)
-static float plain_form_us(const PlainForm& f, int m, int n, int k, int out_bytes, int cus) {
-  const long tiles = ((m + (long)f.bm - 1) / f.bm) * ((n + (long)f.bn - 1) / f.bn);
-  const long x = (tiles + cus - 1) / cus, rounds = (x + f.occ - 1) / f.occ;
+// mb_out: what the output moves (its own bytes, a residual's, a second output's). Runs on the host before
+// every product: 32-bit divisions only.
+static float plain_form_us(const PlainForm& f, u32 tiles, int ksteps, float mb_b, float mb_out, u32 cus) {
+  const u32 x = (tiles + cus - 1) / cus, rounds = (x + f.occ - 1) / f.occ;
   const float step = f.lat * rounds > f.load * x ? f.lat * rounds : f.load * x;
-  const float work = (k / P_BK) * step + f.per_tile * (x - 1), stream = f.stream * 1e-6f * n * k;
-  return f.start + (work > stream ? work : stream) + f.store * 1e-6f * m * n * out_bytes;
+  const float work = ksteps * step + f.per_tile * (x - 1), stream = f.stream * mb_b;
+  return f.start + (work > stream ? work : stream) + f.store * mb_out;
 }
 
 // Whether uwc_gemm_plain_any takes the product: whole k steps, 16-byte output rows (and residual
@@ -641,14 +641,15 @@ bool uwc_plain_any_fits(int m, int n, int k, int ldc, const void* out, int out_m
 // ring while a CU has at most one tile and the 2-step one beyond.
 int uwc_plain_form(int m, int n, int k, int out_mode, int out_bytes, int cus) {
   if (out_mode == P_OUT_NONE) return (long)(m / 128) * (n / 128) <= cus ? 0 : 1;
+  const float mb_b = 1e-6f * n * k, mb_out = 1e-6f * m * n * out_bytes;
   int best = 0;
   float best_us = 0.0f;
   for (int i = 0; i < (int)(sizeof(kPlainForms) / sizeof(kPlainForms[0])); i++) {
     const PlainForm& f = kPlainForms[i];
     // a grid of 2^32 threads or more would be cut off without an error (2^28 rows of 16 columns on 16 x 16 tiles)
-    const u64 tiles = (u64)((m + (long)f.bm - 1) / f.bm) * (u64)((n + (long)f.bn - 1) / f.bn);
+    const u64 tiles = (((u64)m + f.bm - 1) >> __builtin_ctz(f.bm)) * (((u64)n + f.bn - 1) >> __builtin_ctz(f.bn));
     if (i > 0 && tiles * P_THREADS > 0xFFFFFFFFull) continue;
-    const float us = plain_form_us(f, m, n, k, out_bytes, cus);
+    const float us = plain_form_us(f, tiles < 0xFFFFFFFFull ? (u32)tiles : 0xFFFFFFFFu, k / P_BK, mb_b, mb_out, (u32)cus);
     if (i == 0 || us < best_us) best = i, best_us = us;
   }
   return best;
