@@ -855,16 +855,16 @@ def summarize_linears_traffic(fetch_csv, write_csv, out_path, cmd):
         f.write(f"commands: {cmd}\n")
         f.write(f"calibration factors: FETCH_SIZE {res[cases[0][0]]['FETCH_SIZE'][0]:.4f}, WRITE_SIZE "
                 f"{res[cases[0][0]]['WRITE_SIZE'][0]:.4f}\n\n")
-        f.write(f"{'case':34s} {'kernel':44s} {'read MB':>9s} {'write MB':>9s} {'total MB':>9s} {'algo MB':>9s} {'ratio':>6s}\n")
+        f.write(f"{'case':34s} {'kernel':56s} {'read MB':>9s} {'write MB':>9s} {'total MB':>9s} {'algo MB':>9s} {'ratio':>6s}\n")
         for name, m, n, k, what, byt in cases:
             fr, wr = res[name]["FETCH_SIZE"][1], res[name]["WRITE_SIZE"][1]
             for kn in sorted(set(fr) | set(wr)):
                 rd, wt = fr.get(kn, 0.0), wr.get(kn, 0.0)
-                f.write(f"{name:34s} {kn[:44]:44s} {rd / 1e6:9.2f} {wt / 1e6:9.2f} {(rd + wt) / 1e6:9.2f} "
+                f.write(f"{name:34s} {kn[:56]:56s} {rd / 1e6:9.2f} {wt / 1e6:9.2f} {(rd + wt) / 1e6:9.2f} "
                         f"{byt / 1e6:9.2f} {(rd + wt) / byt:6.2f}\n")
         f.write("\nalgo MB: W + X + fp32 out + scales for the GEMMs (uwc_igemm_dequant_f32); fp32 in + int8 out + "
                 "scales for quant_act. ratio > 1: bytes fetched or written beyond the algorithmic ones (e.g. the "
-                "skinny kernels' X broadcast to every workgroup, or W rows read twice through L2).\n")
+                "X read by every XCD's workgroups, or W rows read twice through L2).\n")
     print(open(out_path).read())
 
 
@@ -1064,13 +1064,13 @@ def summarize_e2e_trace(stats_csv, out_path, cmd):
             name = re.sub(r"\(.*", "", r["Name"].replace("(anonymous namespace)::", ""))[:58]
             f.write(f"{name:58s} {int(r['Calls']):6d} {float(r['AverageNs']) / 1e3:9.2f} "
                     f"{float(r['TotalDurationNs']) / 3e6:8.2f} {float(r['Percentage']):5.1f}%\n")
-        f.write("\nPer forward: 28 x (rmsnorm_quant_wave_kernel x 2, noisy_gemm256_kernel<false, false, 1, true> "
+        f.write("\nPer forward: 28 x (rmsnorm_quant_regs_kernel x 2, noisy_gemm256_kernel<false, false, 1, true> "
                 "(the persistent multi-tile form) for qkv and gate_up, noisy_gemm256_kernel<false, false, 4, false> for "
                 "o and down (dequant and residual add in the epilogue), qkv_post_kernel, the stored-exponentials "
                 "attention in two launches (attn_rowmax_kernel: the row maxima; attention_kernel<128, true>: the "
                 "exact sums with the exponentials stored, then P x V from them), quant_act_dgroup_kernel, "
-                "swiglu_quant_wave_kernel), then one batched set of sha_* launches for all 28 layers' stage-output "
-                "roots (sha_block_leaves, sha_row_leaf_quad, sha_group, sha_tree), rmsnorm_quant + the lm_head GEMM "
+                "swiglu_quant_regs_kernel), then one batched set of sha_* launches for all 28 layers' stage-output "
+                "roots (sha_block_leaves, sha_row_tree, sha_group, sha_tree), rmsnorm_quant + the lm_head GEMM "
                 "(256x256 tiles + a 128-wide column tail) + its fp32 dequant (dequant4_kernel) + the logits' Merkle root "
                 "(sha_block_leaves, sha_row_tree, sha_group, sha_tree); ms/fwd = total / 3 (the buffer copies and "
                 "the random-number and scaling kernels are model set-up and the oracle's weight copies, outside the "
@@ -1137,7 +1137,7 @@ def summarize_linears_trace(trace_csv, out_path, cmd):
         f.write("rocprofv3 kernel trace, graph-timed linears of bench.py (configs[1] at M=2048, configs[0], "
                 "Llama-3.1-8B decode at M=1, 8, 32; weights rotated over > 1.2 GB)\n")
         f.write(f"command: {cmd}\n\n")
-        f.write(f"{'shape':44s} {'kernel':44s} {'grid':>6s} {'lds':>7s} {'calls':>6s} {'avg_us':>8s} {'min_us':>8s} "
+        f.write(f"{'shape':44s} {'kernel':56s} {'grid':>6s} {'lds':>7s} {'calls':>6s} {'avg_us':>8s} {'min_us':>8s} "
                 f"{'max_us':>8s}\n")
         for lab, run in zip(LINEAR_LABELS, timed):
             if run is None:
@@ -1145,12 +1145,12 @@ def summarize_linears_trace(trace_csv, out_path, cmd):
             per = {}
             for r in run:
                 name = r["Kernel_Name"].replace("(anonymous namespace)::", "")
-                key = (re.sub(r"\(.*", "", name)[:44], r.get("Grid_Size_X", ""), r.get("LDS_Block_Size", ""))
+                key = (re.sub(r"\(.*", "", name)[:56], r.get("Grid_Size_X", ""), r.get("LDS_Block_Size", ""))
                 per.setdefault(key, []).append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
             for (kn, grid, lds), xs in per.items():
-                f.write(f"{lab[:44]:44s} {kn:44s} {grid:>6s} {lds:>7s} {len(xs):6d} {sum(xs) / len(xs):8.2f} "
+                f.write(f"{lab[:44]:44s} {kn:56s} {grid:>6s} {lds:>7s} {len(xs):6d} {sum(xs) / len(xs):8.2f} "
                         f"{min(xs):8.2f} {max(xs):8.2f}\n")
-        f.write("\ngrid = work-items (workgroups x 640 for skinny_dma_kernel); kernel durations exclude the "
+        f.write("\ngrid = work-items (workgroups x 256; x 128 for wave_gemm_kernel<..., 2, ...>); kernel durations exclude the "
                 "~1.8 us launch gap between dependent graph nodes that the bench's per-launch figures include.\n")
     print(open(out_path).read())
 

@@ -117,8 +117,9 @@ int uwc_igemm_dequant_f32(const int8_t* A, const int8_t* B, int m, int n, int k,
                           float* Y, hipStream_t stream);
 
 /* Y = fadd(x, fmul(fmul(f32(A * B^T), sx[i]), sw[j])) (fp32 m x n, rows of stride n): the exact
- * GEMM with the dequant and the residual add in its epilogue where the 256 x 256 tiles take the
- * shape, else the dequantized product followed by the residual pass; the same bits either way.
+ * GEMM with the dequant and the residual add in its epilogue where the 256 x 256 tiles or the plain
+ * kernels take the shape (k % 128 == 0, n % 4 == 0, 16-byte aligned), else the dequantized product
+ * followed by the residual pass; the same bits either way.
  * Y must not overlap x.
  * Replaces DetLinear.int_gemm + detgpu kernels.dequant_residual of the o and down projections:
  * runtime/detrt/qwen3.py:106-126, runtime/detgpu/kernels.py:805-813, runtime/detrt/stage.py:217, 224. */

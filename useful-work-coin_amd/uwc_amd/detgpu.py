@@ -183,8 +183,8 @@ def dequant_residual(acc, s, sw, x, out=None):
 def linear_residual(lin, q, s, x, out=None):
     """x + fmul(fmul(f32(q @ lin.Wq^T), s), lin.sw): a DetLinear's exact GEMM on pre-quantized rows
     q (N, k) with the dequant and the residual x (N, n) added in one call
-    (uwc_igemm_dequant_residual_f32: in the GEMM's epilogue where its 256 x 256 tiles take the
-    shape), the same bits as dequant_residual(lin.int_gemm(q), s, lin.sw, x). out: an optional
+    (uwc_igemm_dequant_residual_f32: in the GEMM's epilogue where its 256 x 256 tiles or the plain
+    kernels take the shape), the same bits as dequant_residual(lin.int_gemm(q), s, lin.sw, x). out: an optional
     contiguous (N, n) float32 destination that does not overlap x."""
     if lin.mine and lin.mw is not None:
         return dequant_residual(lin.int_gemm(q), s, lin.sw, x, out=out)
@@ -489,7 +489,7 @@ def _layer_call(m, L, x, B, T, out):
 
 def layer_fused(m, L, x: torch.Tensor, B: int, T: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """One decoder layer: x (N, D) float32 -> (N, D) float32, bit-identical to detrt
-    (detgpu/stages.py:154-168); out: optional (N, D) float32 destination, not overlapping x."""
+    (detgpu/stages.py:154-168); out: optional (N, D) float32 destination, which may be x itself."""
     y = _layer_call(m, L, x, B, T, out)
     return y if y is not None else _layer_ops(m, L, x, B, T, out)
 
