@@ -517,6 +517,72 @@ def test_quantizing_row_kernels_widths(dev, rows, k, bs):
     assert np.array_equal(q.cpu().numpy()[pick], rq) and np.array_equal(_u32(s)[pick], _u32(rs))
 
 
+@pytest.mark.parametrize("k", [264, 512, 520, 1024, 1032, 1536, 2048, 2688, 4104, 6144, 14336])
+@pytest.mark.parametrize("rows", [20, 1100])
+def test_row_forms_agree_on_special_values(dev, rows, k):
+    """The register forms against the LDS form (which rows off a 16-byte boundary take) on rows with
+    infinities, NaN, signed zeros, subnormals and the largest values: the same bytes and scales."""
+    from uwc_amd import detgpu, ops
+    g = torch.Generator(device=dev)
+    g.manual_seed(k + rows)
+
+    def off(t):
+        v = torch.empty(t.numel() + 8, dtype=t.dtype, device=dev)[1:1 + t.numel()].view(t.shape)
+        return v.copy_(t)
+
+    def same(got, want):
+        assert torch.equal(got[0], want[0])
+        assert torch.equal(torch.nan_to_num(got[1], nan=-7.0), torch.nan_to_num(want[1], nan=-7.0))
+
+    bs = min(512, k & -k)
+    x = torch.randn((rows, k), device=dev, generator=g)
+    for i, v in enumerate([float("inf"), float("-inf"), float("nan"), -0.0, 1e-45, -1e-40, 3.4e38, -3.4e38, 1e-30]):
+        x[i, (7 * i) % k] = v
+    x[9], x[10], x[11], x[12], x[13] = 0.0, float("nan"), float("inf"), 1e-42, 3e38
+    w = torch.rand(k, device=dev, generator=g)
+    xb = x.to(torch.bfloat16)
+    acc = torch.randint(-2 ** 31, 2 ** 31 - 1, (rows, 2 * k), dtype=torch.int32, device=dev, generator=g)
+    s3 = torch.rand(rows, device=dev, generator=g) * 1e-6
+    s3[:8] = torch.tensor([float("inf"), float("nan"), 0.0, 1e-45, 3e38, 1e30, 1e-30, -1.0])
+    sw = torch.rand(2 * k, device=dev, generator=g)
+    for b in (0, bs):
+        same(detgpu.quant_act(x, b), detgpu.quant_act(off(x), b))
+        same(detgpu.rmsnorm_quant(x, w, 1e-6, b), detgpu.rmsnorm_quant(off(x), w, 1e-6, b))
+        same(detgpu.swiglu_quant(acc, s3, sw, b), detgpu.swiglu_quant(off(acc), s3, sw, b))
+        same(ops.quant_rows_had(xb, b), ops.quant_rows_had(off(xb), b))
+
+
+def test_one_call_paths_replay_from_a_graph(dev):
+    """layer_fused, final_logits and DetLinear captured: every replay, with other work and a
+    synchronization between, equals the eager result on its inputs."""
+    from uwc_amd import detgpu, detrt
+    cfg = dict(D=256, H=4, Hkv=2, hd=64, I=384, L=1, V=512, eps=1e-6, Bs=64, max_pos=70, theta=1e4, arch=0)
+    m = detgpu.DetModel.random(cfg, seed=6, device=dev)
+    L = m.layers[0]
+    lin = detrt.DetLinear.from_quantized(L["qkv"].Wq, L["qkv"].sw, L["qkv"].bs)
+    run = lambda t: (detgpu.layer_fused(m, L, t, 2, 70), *detgpu.final_logits(m, t), lin(t))
+    x = torch.randn((140, 256), device=dev)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        run(x)
+        st.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st):
+            outs = run(x)
+    torch.cuda.synchronize()
+    for seed in range(3):
+        x.copy_(torch.randn((140, 256), generator=torch.Generator().manual_seed(seed)))
+        want = run(x)
+        torch.cuda.synchronize()
+        for o in outs:
+            o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for o, v in zip(outs, want):
+            assert torch.equal(o, v)
+
+
 def test_one_call_paths_take_weights_only_as_they_lie(dev):
     """layer_fused and final_logits over reassigned weights: strided scales give the same rows, a strided
     or float weight is refused as by the op-by-op path, and so are Hadamard blocks that do not divide."""
