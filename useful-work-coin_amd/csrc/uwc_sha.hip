@@ -157,17 +157,19 @@ __device__ void sha_block_leaf(const u32* __restrict__ p, int n, u32 out[8]) {
 
 #define SHA_BLOCK_WORDS 256  // 1 KiB
 
-// One thread per (row, block): the block leaves of every row.
+// One thread per (row, block): the block leaves of every row. Threads past the last block hash it again
+// and store nothing: a wave with idle lanes and few others on its CU takes longer than a full one (20
+// rows of 256 words 60 -> 54 us, 20 of 1024 73 -> 67, 2000 of 256 63 -> 56 with the row trees).
 template <bool VEC>
 __global__ void sha_block_leaves_kernel(const u32* __restrict__ rows, long nrows, int row_words, int nblk,
                                         u32* __restrict__ leaves) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nrows * nblk) return;
-  const long r = i / nblk;
+  const long at = (long)blockIdx.x * blockDim.x + threadIdx.x, last = nrows * nblk - 1;
+  const long i = min(at, last), r = i / nblk;
   const int b = (int)(i - r * nblk);
   const int off = b * SHA_BLOCK_WORDS, n = min(SHA_BLOCK_WORDS, row_words - off);
   u32 h[8];
   sha_block_leaf<VEC>(rows + r * row_words + off, n, h);
+  if (at > last) return;
   uint4* o = reinterpret_cast<uint4*>(leaves + i * 8);
   o[0] = make_uint4(h[0], h[1], h[2], h[3]);
   o[1] = make_uint4(h[4], h[5], h[6], h[7]);
@@ -359,8 +361,8 @@ extern "C" int uwc_sha_row_leaves(const uint32_t* rows, int64_t nrows, int row_w
   // four waves per workgroup, one per SIMD: with two, a CU's workgroups share two of its SIMDs (8192
   // rows of 2048 words 96 -> 61 us, 300 of 151,936 190 -> 149). While the waves are no more than two per
   // CU, workgroups of two spread them over the CUs (20 and 40 rows of 151,936 words 57.2 -> 55.1 us).
-  // Workgroups of one wave do so no better and are slower where lanes run out or end early (4096 rows of
-  // 300 words 51 -> 64 us, 200 of 256 50 -> 56, one of 151,936 51 -> 57).
+  // Workgroups of one wave gain another 1% where every lane runs to the end and lose 20% where half of
+  // them end early (4096 rows of 300 words, with the row trees: 61.8 us, 76.5 at one wave).
   const long waves = (nt + 63) / 64, cus = uwc_cu_count();
   const int threads = waves <= 2 * cus ? 128 : 256;
   const dim3 grid((unsigned)((nt + threads - 1) / threads));
